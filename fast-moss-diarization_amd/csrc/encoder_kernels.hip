@@ -153,18 +153,36 @@ __global__ void __launch_bounds__(256) layernorm_kernel(const void* xv, int ldx,
 // ---------------------------------------------------------------------------
 // Dense bidirectional attention of the encoder (whisper_encoder.rs:44-64) for
 // head_dim 64: q and k arrive already scaled by head_dim^-1/4, so the scores
-// are rd(q . k) with no further scale, the probabilities rd(exp(s - M) / S)
-// with each row's global max M and sum S (softmax_last_dim returns the
-// dtype), and the context rd(P V).  Rounding after normalisation needs M and
-// S first, so each work-group visits its keys twice: pass 1 finds (M, S),
-// pass 2 recomputes the scores and accumulates P V.
+// are q . k with no further scale; context rd(sum_j p_j v_j / sum_j p_j) with
+// p_j = rd(exp(s_j - m)), one pass over the keys with a running reference m
+// per query row (online softmax).
 //
-// One work-group per (64-query tile, head, window), four waves of 16 queries.
-// Keys come in blocks of 64 (K, and in pass 2 V: 8 KiB each), copied global
-// -> LDS by direct-to-LDS loads, double-buffered, the next block in flight
-// while the current one is computed.  S^T = K Q^T puts keys on the MFMA's M
-// side, so the f32 result already sits in the B-operand layout of P^T, and
-// O^T += V^T P^T reads V^T from the row-major V block by LDS transpose reads.
+// Bound by VALU issue: per score half a max, the exponent's fma, v_exp_f32 at
+// a quarter rate and half a packed conversion, against 4.5 MFMA cycles.  The
+// scores stay in f32 (they are never rounded to 16 bits), and sum_j p_j comes
+// from an MFMA against ones over the same rounded p that weigh V.  Visiting
+// the keys twice (p rounded after the division by the final sum) spent about
+// 17 VALU instructions per score and recomputed every score: 16 windows of
+// 1500 positions, 16 heads, bf16: 350 -> 189 us (780 TFLOP/s of the 147
+// GFLOP); one window 40 -> 22.5 us.
+//
+// A window of at most 64 positions is one block: its p are rounded after the
+// division by their sum, as softmax_last_dim returns them.
+//
+// m moves only when a score exceeds it by more than kGrow (log2 units): p then
+// stays below 2^kGrow, far inside f16, and after a row's first block the
+// accumulators are almost never rescaled.  The decision is per row, so a
+// row's result does not depend on which rows share its wave.
+//
+// One work-group per (64 QS queries, head, window), four waves of 16 QS
+// queries; each K or V^T fragment read from LDS feeds QS MFMAs.  Two query
+// sets halve the LDS reads per score; launches whose 128-query grid would
+// leave CUs idle take one (launch_enc_attn).  Keys come in blocks of 64 (K and
+// V: 8 KiB each), copied global -> LDS by direct-to-LDS loads,
+// double-buffered, the next block in flight while the current one is
+// computed.  S^T = K Q^T puts keys on the MFMA's M side, so the f32 result
+// already sits in the B-operand layout of P^T, and O^T += V^T P^T reads V^T
+// from the row-major V block by LDS transpose reads.
 //
 // LDS rows are 128 bytes (64 dims), unpadded; the 16-byte chunk c of key row
 // r sits at chunk position c ^ swk(r) (K) or c ^ swv(r) (V): the K fragment
@@ -198,20 +216,12 @@ __device__ __forceinline__ uint32_t pack2(float a, float b) {
     return __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2){a, b}, f16x2));
   }
 }
-template <int A>
-__device__ __forceinline__ f32x2 unpack2(uint32_t v) {
-  if constexpr (A == ACT_BF16) {
-    return f32x2{__builtin_bit_cast(float, v << 16), __builtin_bit_cast(float, v & 0xffff0000u)};
-  } else {
-    typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
-    return __builtin_convertvector(__builtin_bit_cast(f16x2, v), f32x2);
-  }
-}
 
 constexpr float kLog2e = 1.4426950408889634f;
+constexpr float kGrow = 8.f;   // log2 units a row's scores may exceed its reference by
 
-template <int A>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2)))
+template <int A, int QS>
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(QS == 2 ? 3 : 4)))
 enc_attn_kernel(EncAttnArgs p) {
   typedef typename ActT<A>::T T;
   constexpr int BLK = EKB * EHD;   // elements of one K or V block
@@ -230,17 +240,18 @@ enc_attn_kernel(EncAttnArgs p) {
   const int h = (lid / nx) % ny;
   const size_t row0 = (size_t)(lid / (nx * ny)) * p.period;
   const uint16_t* base = (const uint16_t*)p.qkv + row0 * p.ld;
-  const int q0 = (lid % nx) * 64 + 16 * w;
+  const int q0 = (lid % nx) * (64 * QS) + 16 * QS * w;
   const int nblk = (p.t + EKB - 1) / EKB;
 
-  // Q^T fragments (B operand): query q0 + qr (rows past t read row t - 1;
-  // their outputs are not stored), dims 32 ks + 8 kg .. + 7.
-  u32x4 qf[2];
-  {
-    const int qrow = min(q0 + qr, p.t - 1);
+  // Q^T fragments (B operand): query q0 + 16 qs + qr (rows past t read row
+  // t - 1; their outputs are not stored), dims 32 ks + 8 kg .. + 7.
+  u32x4 qf[QS][2];
+#pragma unroll
+  for (int qs = 0; qs < QS; ++qs) {
+    const int qrow = min(q0 + 16 * qs + qr, p.t - 1);
 #pragma unroll
     for (int ks = 0; ks < 2; ++ks)
-      qf[ks] = *(const u32x4*)(base + (size_t)qrow * p.ld + h * EHD + ks * 32 + kg * 8);
+      qf[qs][ks] = *(const u32x4*)(base + (size_t)qrow * p.ld + h * EHD + ks * 32 + kg * 8);
   }
 
   // Block copies: 8 wave instructions of 1 KiB (8 key rows) per operand;
@@ -258,8 +269,7 @@ enc_attn_kernel(EncAttnArgs p) {
     vch[i] = (uint32_t)(2 * p.d + h * EHD + ((pc ^ swv(rr)) << 3)) * 2u;
   }
   const uint32_t lk = lds_addr(sK), lv = lds_addr(sV);
-  auto issue = [&](int blk, auto with_v_tag) {
-    constexpr bool WV = decltype(with_v_tag)::value;
+  auto issue = [&](int blk) {
     const int k0 = blk * EKB;
     const uint32_t boff = (uint32_t)(blk & 1) * (BLK * 2);
 #pragma unroll
@@ -267,115 +277,125 @@ enc_attn_kernel(EncAttnArgs p) {
       const uint32_t j = (uint32_t)(2 * wu + i);
       const uint32_t roff = (uint32_t)min(k0 + crow[i], p.t - 1) * (uint32_t)p.ld * 2u;
       lds_copy16(base, roff + kch[i], lk + boff + j * 1024u);
-      if constexpr (WV) lds_copy16(base, roff + vch[i], lv + boff + j * 1024u);
+      lds_copy16(base, roff + vch[i], lv + boff + j * 1024u);
     }
   };
 
-  // Raw S^T of sub-block mt (keys 16 mt .. 16 mt + 15 of the block).
-  auto qk = [&](const uint16_t* kb, int mt) {
-    f32x4 sv = {0.f, 0.f, 0.f, 0.f};
-    const int r = 16 * mt + qr;
+  // m: the row's reference (raw score units), in every lane of the row.
+  // ls: MFMA accumulator of the row's sum of p (every element holds it; only
+  // element 0 is kept in step with m).
+  float m[QS], ml2[QS];
+  f32x4 o[QS][4], ls[QS];
 #pragma unroll
-    for (int ks = 0; ks < 2; ++ks) {
-      const u32x4 ka = *(const u32x4*)&kb[r * EHD + (((4 * ks + kg) ^ swk(r)) << 3)];
-      sv = mfma16<A>(ka, qf[ks], sv);
-    }
-    return sv;
-  };
-  // rd(q . k) in place; with MASKED (the last block, when t is not a
-  // multiple of the block), keys at or past t become -inf.  The flag is a
-  // compile-time one so that full blocks run without branches and their
-  // four sub-blocks' products and roundings can interleave.
-  auto round_mask = [&](f32x4& sv, int kbase, auto masked_tag) {
-    if constexpr (A == ACT_BF16) {
+  for (int qs = 0; qs < QS; ++qs) {
+    m[qs] = -INFINITY;
+    ml2[qs] = 0.f;
+    ls[qs] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-      for (int i = 0; i < 4; ++i) sv[i] = rd<A>(sv[i]);   // one conversion each
-    } else {
+    for (int i = 0; i < 4; ++i) o[qs][i] = f32x4{0.f, 0.f, 0.f, 0.f};
+  }
+  const uint32_t one2 = pack2<A>(1.f, 1.f);
+  const u32x4 ones = u32x4{one2, one2, one2, one2};
+  typedef short s16x4 __attribute__((ext_vector_type(4)));
+  typedef __attribute__((address_space(3))) s16x4 lds_s16x4;
+  const int ts = lane & 15;
+  // This lane's fragment positions in a block (elements): K row qr, chunk
+  // 4 ks + kg (row 16 mt + qr: + 16 mt rows, same swizzle); V^T pieces of key
+  // 4 kg + ts / 4 at dims 16 dt + 4 (ts % 4) (keys 16 and 32 further on: same
+  // swizzle).
+  int ke[2], ve[4];
 #pragma unroll
-      for (int i = 0; i < 4; i += 2) {
-        const f32x2 v = unpack2<A>(pack2<A>(sv[i], sv[i + 1]));
-        sv[i] = v.x;
-        sv[i + 1] = v.y;
+  for (int ks = 0; ks < 2; ++ks) ke[ks] = qr * EHD + (((4 * ks + kg) ^ swk(qr)) << 3);
+#pragma unroll
+  for (int dt = 0; dt < 4; ++dt) {
+    const int key = 4 * kg + (ts >> 2);
+    ve[dt] = key * EHD + (((2 * dt + ((ts & 3) >> 1)) ^ swv(key)) << 3) + 4 * (ts & 1);
+  }
+
+  auto block = [&](int blk, auto masked_tag) {
+    const uint16_t* kb = sK + (blk & 1) * BLK;
+    const uint16_t* vb = sV + (blk & 1) * BLK;
+    // S^T of sub-block mt: keys 16 mt + 4 kg + i of the block
+    f32x4 sv[QS][4];
+#pragma unroll
+    for (int mt = 0; mt < 4; ++mt) {
+      u32x4 ka[2];
+#pragma unroll
+      for (int ks = 0; ks < 2; ++ks) ka[ks] = *(const u32x4*)&kb[ke[ks] + 16 * mt * EHD];
+#pragma unroll
+      for (int qs = 0; qs < QS; ++qs) {
+        sv[qs][mt] = mfma16<A>(ka[0], qf[qs][0], f32x4{0.f, 0.f, 0.f, 0.f});
+        sv[qs][mt] = mfma16<A>(ka[1], qf[qs][1], sv[qs][mt]);
       }
     }
     if constexpr (decltype(masked_tag)::value) {
 #pragma unroll
-      for (int i = 0; i < 4; ++i)
-        if (kbase + 4 * kg + i >= p.t) sv[i] = -INFINITY;
+      for (int qs = 0; qs < QS; ++qs)
+#pragma unroll
+        for (int mt = 0; mt < 4; ++mt)
+#pragma unroll
+          for (int i = 0; i < 4; ++i)
+            if (blk * EKB + 16 * mt + 4 * kg + i >= p.t) sv[qs][mt][i] = -INFINITY;
     }
-  };
-
-  // Pass 1: max and sum of exp of each query row (each lane covers 16 keys
-  // of a block; the four lanes of a row merge at the end).
-  float m = -INFINITY, l = 0.f;
-  auto pass1_block = [&](int blk, auto masked_tag) {
-    const uint16_t* kb = sK + (blk & 1) * BLK;
-    f32x4 sv[4];
+    if (decltype(masked_tag)::value && nblk == 1) {
+      // The row's max and sum are known before any p is rounded: p = rd(exp(s -
+      // M) / S) over rounded scores, as softmax_last_dim returns it.
 #pragma unroll
-    for (int mt = 0; mt < 4; ++mt) sv[mt] = qk(kb, mt);
+      for (int qs = 0; qs < QS; ++qs) {
+        float M = -INFINITY, S = 0.f;
 #pragma unroll
-    for (int mt = 0; mt < 4; ++mt) round_mask(sv[mt], blk * EKB + 16 * mt, masked_tag);
-    float bm = -INFINITY;
+        for (int e = 0; e < 16; ++e) {
+          sv[qs][e >> 2][e & 3] = rd<A>(sv[qs][e >> 2][e & 3]);
+          M = fmaxf(M, sv[qs][e >> 2][e & 3]);
+        }
+        M = fmaxf(M, __shfl_xor(M, 16));
+        M = fmaxf(M, __shfl_xor(M, 32));
+        ml2[qs] = (M == -INFINITY ? 0.f : M) * kLog2e;
 #pragma unroll
-    for (int mt = 0; mt < 4; ++mt)
+        for (int e = 0; e < 16; ++e) S += __builtin_amdgcn_exp2f(fmaf(sv[qs][e >> 2][e & 3], kLog2e, -ml2[qs]));
+        S += __shfl_xor(S, 16);
+        S += __shfl_xor(S, 32);
+        ml2[qs] += __log2f(S > 0.f ? S : 1.f);
+      }
+    } else {
+      float bm[QS];
+      bool grow = false;
 #pragma unroll
-      for (int i = 0; i < 4; ++i) bm = fmaxf(bm, sv[mt][i]);
-    const float mn = fmaxf(m, bm);
-    const float ml2 = (mn == -INFINITY ? 0.f : mn) * kLog2e;
-    float e = l * __builtin_amdgcn_exp2f(fmaf(m, kLog2e, -ml2));
+      for (int qs = 0; qs < QS; ++qs) {
+        bm[qs] = sv[qs][0][0];
 #pragma unroll
-    for (int mt = 0; mt < 4; ++mt)
+        for (int e = 1; e < 16; ++e) bm[qs] = fmaxf(bm[qs], sv[qs][e >> 2][e & 3]);
+        grow |= fmaf(bm[qs], kLog2e, -ml2[qs]) > kGrow || m[qs] == -INFINITY;
+      }
+      if (__any(grow)) {
 #pragma unroll
-      for (int i = 0; i < 4; ++i) e += __builtin_amdgcn_exp2f(fmaf(sv[mt][i], kLog2e, -ml2));
-    m = mn;
-    l = e;
-  };
-  issue(0, std::false_type{});
-  for (int blk = 0; blk < nblk; ++blk) {
-    wait_vm<0>();      // this block's copies (the only ones in flight) have landed
-    barrier_lds();     // for every wave; and block blk - 1's buffer is free
-    if (blk + 1 < nblk) issue(blk + 1, std::false_type{});
-    if ((blk + 1) * EKB > p.t) pass1_block(blk, std::true_type{});
-    else pass1_block(blk, std::false_type{});
-  }
+        for (int qs = 0; qs < QS; ++qs) {
+          float rm = fmaxf(bm[qs], __shfl_xor(bm[qs], 16));
+          rm = fmaxf(rm, __shfl_xor(rm, 32));
+          // per row: every lane of the row decides alike
+          const bool move = fmaf(rm, kLog2e, -ml2[qs]) > kGrow || m[qs] == -INFINITY;
+          const float mn = move ? fmaxf(rm, m[qs]) : m[qs];
+          const float nl2 = (mn == -INFINITY ? 0.f : mn) * kLog2e;
+          const float c = move ? __builtin_amdgcn_exp2f(fmaf(m[qs], kLog2e, -nl2)) : 1.f;
+          m[qs] = mn;
+          ml2[qs] = nl2;
+          ls[qs][0] *= c;
 #pragma unroll
-  for (int off = 16; off <= 32; off <<= 1) {
-    const float mo = __shfl_xor(m, off), lo = __shfl_xor(l, off);
-    const float mn = fmaxf(m, mo);
-    const float mref = mn == -INFINITY ? 0.f : mn;
-    l = l * __expf(m - mref) + lo * __expf(mo - mref);
-    m = mn;
-  }
-  // exp(s - M) / S as one power of two, exp2(s log2 e - (M log2 e + log2 S)):
-  // the division folds into the exponent's offset (one multiply less per
-  // score; a few f32 ulps before the probability's rounding)
-  const float mlog = fmaf(m == -INFINITY ? 0.f : m, kLog2e, __log2f(l > 0.f ? l : 1.f));
-  barrier_lds();   // pass 1's last reads of the K buffers precede pass 2's copies
-
-  // Pass 2: p = rd(exp(s - M) / S), O^T += V^T P^T.
-  f32x4 o[4];
-#pragma unroll
-  for (int i = 0; i < 4; ++i) o[i] = f32x4{0.f, 0.f, 0.f, 0.f};
-  typedef short s16x4 __attribute__((ext_vector_type(4)));
-  typedef __attribute__((address_space(3))) s16x4 lds_s16x4;
-  const int ts = lane & 15;
-  auto pass2_block = [&](int blk, auto masked_tag) {
-    const uint16_t* kb = sK + (blk & 1) * BLK;
-    const uint16_t* vb = sV + (blk & 1) * BLK;
-    f32x4 sv[4];
-#pragma unroll
-    for (int mt = 0; mt < 4; ++mt) sv[mt] = qk(kb, mt);
-    uint32_t pp[4][2];
-#pragma unroll
-    for (int mt = 0; mt < 4; ++mt) {
-      round_mask(sv[mt], blk * EKB + 16 * mt, masked_tag);
-#pragma unroll
-      for (int i = 0; i < 4; i += 2) {
-        const float e0 = __builtin_amdgcn_exp2f(fmaf(sv[mt][i], kLog2e, -mlog));
-        const float e1 = __builtin_amdgcn_exp2f(fmaf(sv[mt][i + 1], kLog2e, -mlog));
-        pp[mt][i / 2] = pack2<A>(e0, e1);
+          for (int dt = 0; dt < 4; ++dt) o[qs][dt] *= c;
+        }
       }
     }
+    uint32_t pp[QS][4][2];
+#pragma unroll
+    for (int mt = 0; mt < 4; ++mt)
+#pragma unroll
+      for (int qs = 0; qs < QS; ++qs)
+#pragma unroll
+        for (int i = 0; i < 4; i += 2) {
+          const float e0 = __builtin_amdgcn_exp2f(fmaf(sv[qs][mt][i], kLog2e, -ml2[qs]));
+          const float e1 = __builtin_amdgcn_exp2f(fmaf(sv[qs][mt][i + 1], kLog2e, -ml2[qs]));
+          pp[qs][mt][i / 2] = pack2<A>(e0, e1);
+        }
     // keys 32 hb .. 32 hb + 31: k-slot s of lane group kg holds key 32 hb +
     // 4 kg + s (s < 4) or 32 hb + 16 + 4 kg + (s - 4), where S^T put them.
     // For the V^T operand (row = dim 16 dt + ts), lane ts supplies the
@@ -383,39 +403,51 @@ enc_attn_kernel(EncAttnArgs p) {
     // read) at dims 16 dt + 4 (ts % 4) .. + 3.
 #pragma unroll
     for (int hb = 0; hb < 2; ++hb) {
-      const u32x4 pb = u32x4{pp[2 * hb][0], pp[2 * hb][1], pp[2 * hb + 1][0], pp[2 * hb + 1][1]};
-      const int key1 = 32 * hb + 4 * kg + (ts >> 2);
-      const int sw = swv(key1);   // = swv(key1 + 16)
+      u32x4 pb[QS];
+#pragma unroll
+      for (int qs = 0; qs < QS; ++qs)
+        pb[qs] = u32x4{pp[qs][2 * hb][0], pp[qs][2 * hb][1], pp[qs][2 * hb + 1][0], pp[qs][2 * hb + 1][1]};
       s16x4 r1[4], r2[4];
 #pragma unroll
       for (int dt = 0; dt < 4; ++dt) {
-        const int e = (((2 * dt + ((ts & 3) >> 1)) ^ sw) << 3) + 4 * (ts & 1);
-        r1[dt] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(vb + key1 * EHD + e));
-        r2[dt] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(vb + (key1 + 16) * EHD + e));
+        r1[dt] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(vb + ve[dt] + 32 * hb * EHD));
+        r2[dt] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(vb + ve[dt] + (32 * hb + 16) * EHD));
       }
+#pragma unroll
+      for (int qs = 0; qs < QS; ++qs) ls[qs] = mfma16<A>(ones, pb[qs], ls[qs]);
 #pragma unroll
       for (int dt = 0; dt < 4; ++dt) {
         const u32x4 va =
             __builtin_bit_cast(u32x4, __builtin_shufflevector(r1[dt], r2[dt], 0, 1, 2, 3, 4, 5, 6, 7));
-        o[dt] = mfma16<A>(va, pb, o[dt]);
+#pragma unroll
+        for (int qs = 0; qs < QS; ++qs) o[qs][dt] = mfma16<A>(va, pb[qs], o[qs][dt]);
       }
     }
   };
-  issue(0, std::true_type{});
-  for (int blk = 0; blk < nblk; ++blk) {
+  issue(0);
+  const int nfull = nblk == 1 ? 0 : p.t / EKB;   // blocks that run unmasked
+  for (int blk = 0; blk < nfull; ++blk) {
+    wait_vm<0>();      // this block's copies (the only ones in flight) have landed
+    barrier_lds();     // for every wave; and block blk - 1's buffers are free
+    if (blk + 1 < nblk) issue(blk + 1);
+    block(blk, std::false_type{});
+  }
+  if (nfull < nblk) {
     wait_vm<0>();
     barrier_lds();
-    if (blk + 1 < nblk) issue(blk + 1, std::true_type{});
-    if ((blk + 1) * EKB > p.t) pass2_block(blk, std::true_type{});
-    else pass2_block(blk, std::false_type{});
+    block(nfull, std::true_type{});
   }
-  // Context rd(O): lane holds dims 16 dt + 4 kg .. + 3 of query q0 + qr.
-  if (q0 + qr < p.t) {
-    T* out = (T*)p.out + (row0 + q0 + qr) * p.ldo + h * EHD;
+  // Context rd(O / sum): lane holds dims 16 dt + 4 kg .. + 3 of query row qr.
+#pragma unroll
+  for (int qs = 0; qs < QS; ++qs) {
+    const int q = q0 + 16 * qs + qr;
+    if (q >= p.t) continue;
+    const float inv = nblk == 1 ? 1.f : 1.f / (ls[qs][0] > 0.f ? ls[qs][0] : 1.f);
+    T* out = (T*)p.out + (row0 + q) * p.ldo + h * EHD;
 #pragma unroll
     for (int dt = 0; dt < 4; ++dt)
-      *(uint2*)&out[16 * dt + 4 * kg] =
-          uint2{pack2<A>(o[dt][0], o[dt][1]), pack2<A>(o[dt][2], o[dt][3])};
+      *(uint2*)&out[16 * dt + 4 * kg] = uint2{pack2<A>(o[qs][dt][0] * inv, o[qs][dt][1] * inv),
+                                              pack2<A>(o[qs][dt][2] * inv, o[qs][dt][3] * inv)};
   }
 }
 
@@ -517,6 +549,20 @@ hipError_t launch_layernorm(int act, const void* x, int ldx, const void* w, cons
   return hipGetLastError();
 }
 
+// 128-query tiles (two query sets per wave) once their grid gives each of the
+// 256 CUs two work-groups, else 64-query tiles (a whole layer at 16 heads of
+// 1500 positions, 64- against 128-query tiles: 2 windows, 384 work-groups of
+// 128 queries, 192.2 / 196.0 us; 3 windows 265.5 / 266.3; 4 windows 314.7 /
+// 310.3; 16 windows 956 / 930).
+template <int A>
+static void launch_enc_attn16(const EncAttnArgs& a, int heads, int windows, hipStream_t s) {
+  const int tiles2 = (a.t + 127) / 128;
+  if ((int64_t)tiles2 * heads * windows >= 512)
+    hipLaunchKernelGGL((enc_attn_kernel<A, 2>), dim3(tiles2, heads, windows), dim3(256), 0, s, a);
+  else
+    hipLaunchKernelGGL((enc_attn_kernel<A, 1>), dim3((a.t + 63) / 64, heads, windows), dim3(256), 0, s, a);
+}
+
 hipError_t launch_enc_attn(int act, const EncAttnArgs& a, int heads, int windows, hipStream_t s) {
   if (windows <= 0 || a.t <= 0) return hipSuccess;
   if (heads <= 0 || a.d != heads * EHD || a.period < a.t || a.ld % 8 || a.ldo % 4)
@@ -525,12 +571,8 @@ hipError_t launch_enc_attn(int act, const EncAttnArgs& a, int heads, int windows
     case ACT_F32:
       hipLaunchKernelGGL(enc_attn_f32_kernel, dim3(a.t, heads, windows), dim3(64), 0, s, a);
       break;
-    case ACT_F16:
-      hipLaunchKernelGGL(enc_attn_kernel<ACT_F16>, dim3((a.t + 63) / 64, heads, windows), dim3(256), 0, s, a);
-      break;
-    case ACT_BF16:
-      hipLaunchKernelGGL(enc_attn_kernel<ACT_BF16>, dim3((a.t + 63) / 64, heads, windows), dim3(256), 0, s, a);
-      break;
+    case ACT_F16: launch_enc_attn16<ACT_F16>(a, heads, windows, s); break;
+    case ACT_BF16: launch_enc_attn16<ACT_BF16>(a, heads, windows, s); break;
     default: return hipErrorInvalidValue;
   }
   return hipGetLastError();

@@ -267,3 +267,33 @@ def test_windows_are_independent_of_the_batch(fmd, orc):
     for i in (0, 5, 11):
         alone = gpu.forward(mel[i:i + 1])
         assert np.array_equal(together[i], alone[0]), i
+
+
+@pytest.mark.parametrize("t,windows", [(1, 2), (63, 2), (64, 2), (65, 256), (128, 2), (130, 128)])
+def test_attention_key_blocks_and_growing_scores(fmd, orc, t, windows):
+    """Window lengths around the 64-key blocks, on both query tilings (two
+    heads and 256 or 128 windows reach the 128-query tiles).  q and k
+    projections are 1.5 times the identity, and the positions of each 64-key
+    block share a direction, so a row's scores are about 1.5^2 64 / 8 = 18
+    inside its own block and within a few units of 0 outside: rows of later
+    blocks meet scores e^18 above everything before them, and the running
+    reference has to move.  Bars as above; and a window alone gives the bits it
+    has in the batch."""
+    print(f"[gpu] encoder attention t={t} windows={windows}", flush=True)
+    cfg = acfg(fmd, layers=1, max_source_positions=256)
+    w = fmd.synthetic_audio_weights(cfg, seed=21)
+    p = "model.whisper_encoder.layers.0.self_attn."
+    for n in ("q_proj", "k_proj"):
+        w[p + n + ".weight"] = (1.5 * np.eye(128)).astype(np.float32)
+    gpu = fmd.AudioEncoder(cfg, "int8").load(w)
+    ref = orc.OracleEncoder(cfg, OP["f16"]).load(w)
+    rng = np.random.default_rng(22 + t)
+    own = rng.standard_normal((windows, (t + 63) // 64, 128))
+    x = np.repeat(own, 64, axis=1)[:, :t] + 0.1 * rng.standard_normal((windows, t, 128))
+    x = orc.round_to(x.astype(np.float32), OP["f16"])
+    got = gpu.layers(from_f32(x, "f16", orc), 0, 1)
+    assert np.all(np.isfinite(to_f32(got, "f16")))
+    check(to_f32(got, "f16"), ref.layers(x, 0, 1), "f16", f"layer t={t}")
+    for i in (0, windows - 1):
+        alone = gpu.layers(from_f32(x[i:i + 1], "f16", orc), 0, 1)
+        assert np.array_equal(alone[0], got[i]), i
