@@ -1,18 +1,17 @@
 // Prefill projections: Y = X W^T for many rows on the MFMA units.
 //
-// Block tiles of 64, 128 or 256 rows x 128 weight rows, four waves in a 2x2
-// arrangement, MFMA 16x16x32, B fragments from the tiled weight layout
-// shared with the decode GEMV (one 16-byte piece per lane per 16x32
-// fragment):
-// - dense 16-bit weights (gemm_dma_kernel, 64, 128 or 256 rows): both
-//   operands go global -> LDS by direct-to-LDS loads through a ring of 32-k
-//   stages; waves hold 32 x 64, 64 x 64 or 128 x 64.
-// - 64 rows (gemm16_kernel), for the smallest grids and for Q8_0: K step 64,
-//   X staged global -> registers -> LDS, double-buffered
-//   with one barrier per K step (row pitch padded to 72 elements so the
-//   MFMA-order 16-byte reads are bank-conflict free); dense weights take the
-//   same route, Q8_0 fragments are read straight from global memory one K
-//   step ahead; waves hold 32 x 64.
+// Four waves in a 2x2 arrangement, MFMA 16x16x32, B fragments from the tiled
+// weight layout shared with the decode GEMV (one 16-byte piece per lane per
+// 16x32 fragment):
+// - small grids (gemm_small_kernel): tiles of 32 to 128 rows x 32 to 128
+//   columns, dense or Q8_0, chosen so that the grid covers the CUs (try_small);
+// - dense 16-bit weights (gemm_dma_kernel, 64, 128 or 256 rows x 128 columns):
+//   both operands go global -> LDS by direct-to-LDS loads through a ring of
+//   32-k stages; waves hold 32 x 64, 64 x 64 or 128 x 64;
+// - Q8_0 (gemm_q8_kernel, 64 rows x 128 columns): K step 64, X staged global ->
+//   registers -> LDS, double-buffered with one barrier per K step (row pitch
+//   padded to 72 elements so the MFMA-order 16-byte reads are bank-conflict
+//   free), fragments read straight from global memory one K step ahead.
 // Every global load is unconditional (out-of-range rows and tiles read
 // clamped addresses), so no wait depends on a branch.  Work-groups are
 // mapped to tiles over an XCD grid chosen per shape (see tile_of).  Q8_0
@@ -21,7 +20,6 @@
 //
 // Reference: Linear::forward / FusedLinear::forward (linear.rs:29-100) over
 // (b*t, in) rows; call sites qwen3.rs:213, 258, 288-291.
-#include <cstdlib>
 #include <type_traits>
 
 #include "fmd_common.h"
@@ -139,7 +137,7 @@ template <int A, int BMT, int MI>
 __device__ __forceinline__ void rope_epilogue(const GemmArgs& p, const f32x4 (&acc)[MI][4],
                                               typename ActT<A>::T* stg, int m0, int cg,
                                               const RopeRows<BMT>& rr) {
-  static_assert(BMT == 64 || BMT == 128, "rope tiles");
+  static_assert(BMT == 32 || BMT == 64 || BMT == 128, "rope tiles");
   typedef typename ActT<A>::T T;
   constexpr int NJ = BMT / 16;   // rows per 16-lane group
   const RopeArgs& q = p.rope;
@@ -408,19 +406,18 @@ __device__ __forceinline__ void swiglu_staged_epilogue(const GemmArgs& p, const 
     *(u32x4*)(y + (size_t)R * p.ldy) = *(const u32x4*)&stg[R * 64 + ((ch ^ rope_sw(R)) << 3)];
 }
 
-// LB: the work-group's weight block (8 tiles x 64 k) is staged through LDS
-// like X, so each weight byte is fetched once per work-group instead of once
-// per wave column (dense weights only).
-template <int A, int WK, int EPI, int BMT, bool LB>
+// Q8_0 weights (f16 activations) past the small grids: 64 x 128 tiles, K step
+// 64, X staged global -> registers -> LDS, weight fragments and scales read
+// straight from global memory one K step ahead.  The tiles scale each block's
+// product in f32 on the VALU, so their accumulators live in VGPRs.
+template <int EPI>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2)))
-gemm16_kernel(GemmArgs p) {
+gemm_q8_kernel(GemmArgs p) {
+  constexpr int A = ACT_F16, BMT = 64;
   typedef typename ActT<A>::T T;
-  static_assert(!LB || WK == WK_DENSE, "LDS-staged weights are dense only");
   constexpr int MI = BMT / 32;   // 16-row fragments per wave (waves are 2 x 2)
   constexpr int NA = BMT / 32;   // 16-byte pieces of the X tile per thread
   __shared__ uint16_t sA[2 * BMT * LDA];
-  // [buffer][local tile 0..7][chunk 0..1][64 lanes][8], B-operand lane order
-  __shared__ uint16_t sB[LB ? 2 * 8 * 2 * 512 : 1];
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
   const int wm = w >> 1, wn = w & 1;
   const int K = p.W.in, ntiles = p.W.out / 16;
@@ -475,60 +472,16 @@ gemm16_kernel(GemmArgs p) {
       *(u32x4*)&sA[buf * BMT * LDA + r * LDA + c * 8] = ra[set][i];
     }
   };
-  // LB staging: thread piece i is local tile lt = 2 i + threadIdx.x / 128
-  // (wave column lt / 4, fragment lt % 4), chunk (threadIdx.x / 64) & 1 and
-  // lane threadIdx.x & 63 of that 1 KiB fragment.
-  int gtile[LB ? 4 : 1];
-  if constexpr (LB) {
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int lt = 2 * i + (threadIdx.x >> 7);
-      const int tl = wave_tile<EPI>(cg, ntiles, lt >> 2, lt & 3);
-      const bool ok = (EPI == EPI_SWIGLU) ? (cg * 4 + (lt >> 2) * 2 + (lt & 1)) < ntiles / 2
-                                          : tl < ntiles;
-      gtile[i] = ok ? tl : ntiles - 1;
-    }
-  }
-  u32x4 rg[LB ? 2 : 1][LB ? 4 : 1];
-  auto load_bg = [&](int kt, int set) {
-    if constexpr (LB) {
-      const int c = (threadIdx.x >> 6) & 1;
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const uint32_t ch = (uint32_t)gtile[i] * (K / 32) + 2 * kt + c;
-        rg[set][i] = ld16(p.W.w, (ch * 64 + lane) * 16u);
-      }
-    }
-  };
-  auto store_bg = [&](int buf, int set) {
-    if constexpr (LB) {
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int piece = threadIdx.x + 256 * i;  // (lt, c, lane) in LDS order
-        *(u32x4*)&sB[buf * 8192 + piece * 8] = rg[set][i];
-      }
-    }
-  };
-  constexpr int NCH = (WK == WK_Q8) ? 1 : 2;  // weight chunks per tile per K step
   // B fragments, double-buffered by step parity: step kt reads set kt & 1,
   // which was loaded during step kt - 1, and loads set (kt + 1) & 1.
-  u32x4 rb[2][4][NCH];
+  u32x4 rb[2][4];
   uint32_t rs[2][4];
   auto load_b = [&](int kt, int set) {
-    if constexpr (LB) return;
 #pragma unroll
     for (int ni = 0; ni < 4; ++ni) {
-      if constexpr (WK == WK_Q8) {
-        const uint32_t ch = (uint32_t)ltile[ni] * (K / 64) + kt;
-        rb[set][ni][0] = ld16(p.W.w, (ch * 64 + lane) * 16u);
-        rs[set][ni] = ld4(p.W.sc, (ch * 16 + row) * 4u);
-      } else {
-#pragma unroll
-        for (int c = 0; c < 2; ++c) {
-          const uint32_t ch = (uint32_t)ltile[ni] * (K / 32) + 2 * kt + c;
-          rb[set][ni][c] = ld16(p.W.w, (ch * 64 + lane) * 16u);
-        }
-      }
+      const uint32_t ch = (uint32_t)ltile[ni] * (K / 64) + kt;
+      rb[set][ni] = ld16(p.W.w, (ch * 64 + lane) * 16u);
+      rs[set][ni] = ld4(p.W.sc, (ch * 16 + row) * 4u);
     }
   };
 
@@ -549,31 +502,18 @@ gemm16_kernel(GemmArgs p) {
   const int KT = K / BK;
   load_a(0, 0);
   load_b(0, 0);
-  load_bg(0, 0);
   load_a(min(1, KT - 1), 1);
-  load_bg(min(1, KT - 1), 1);
   store_a(0, 0);
-  store_bg(0, 0);
   load_a(min(2, KT - 1), 0);
-  load_bg(min(2, KT - 1), 0);
   __syncthreads();
   auto step = [&](auto par, int kt) {
     constexpr int P = decltype(par)::value;
-    u32x4 cb[4][NCH];
+    u32x4 cb[4];
     uint32_t cs[4];
-    if constexpr (LB) {
 #pragma unroll
-      for (int ni = 0; ni < 4; ++ni)
-#pragma unroll
-        for (int c = 0; c < NCH; ++c)
-          cb[ni][c] = *(const u32x4*)&sB[P * 8192 + ((wn * 4 + ni) * 2 + c) * 512 + lane * 8];
-    } else {
-#pragma unroll
-      for (int ni = 0; ni < 4; ++ni) {
-#pragma unroll
-        for (int c = 0; c < NCH; ++c) cb[ni][c] = rb[P][ni][c];
-        cs[ni] = rs[P][ni];
-      }
+    for (int ni = 0; ni < 4; ++ni) {
+      cb[ni] = rb[P][ni];
+      cs[ni] = rs[P][ni];
     }
     load_b(min(kt + 1, KT - 1), P ^ 1);
     const uint16_t* a = sA + P * BMT * LDA;
@@ -585,31 +525,21 @@ gemm16_kernel(GemmArgs p) {
         fa[mi][ks] = *(const u32x4*)&a[(wm * (BMT / 2) + mi * 16 + row) * LDA + ks * 32 + kg * 8];
 #pragma unroll
     for (int ni = 0; ni < 4; ++ni) {
-      if constexpr (WK == WK_Q8) {
-        const u32x4 b0 = q8_to_f16x8(cb[ni][0][0], cb[ni][0][1]);
-        const u32x4 b1 = q8_to_f16x8(cb[ni][0][2], cb[ni][0][3]);
-        const float d0 = f16_to_f32((uint16_t)(cs[ni] & 0xffffu));
-        const float d1 = f16_to_f32((uint16_t)(cs[ni] >> 16));
-        const f32x4 z = {0.f, 0.f, 0.f, 0.f};
+      const u32x4 b0 = q8_to_f16x8(cb[ni][0], cb[ni][1]);
+      const u32x4 b1 = q8_to_f16x8(cb[ni][2], cb[ni][3]);
+      const float d0 = f16_to_f32((uint16_t)(cs[ni] & 0xffffu));
+      const float d1 = f16_to_f32((uint16_t)(cs[ni] >> 16));
+      const f32x4 z = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-        for (int mi = 0; mi < MI; ++mi) {
-          const f32x4 t0 = mfma16<ACT_F16>(fa[mi][0], b0, z);
-          const f32x4 t1 = mfma16<ACT_F16>(fa[mi][1], b1, z);
-          acc[mi][ni] += d0 * t0;
-          acc[mi][ni] += d1 * t1;
-        }
-      } else {
-#pragma unroll
-        for (int mi = 0; mi < MI; ++mi) {
-          acc[mi][ni] = mfma16<A>(fa[mi][0], cb[ni][0], acc[mi][ni]);
-          acc[mi][ni] = mfma16<A>(fa[mi][1], cb[ni][1], acc[mi][ni]);
-        }
+      for (int mi = 0; mi < MI; ++mi) {
+        const f32x4 t0 = mfma16<ACT_F16>(fa[mi][0], b0, z);
+        const f32x4 t1 = mfma16<ACT_F16>(fa[mi][1], b1, z);
+        acc[mi][ni] += d0 * t0;
+        acc[mi][ni] += d1 * t1;
       }
     }
     store_a(P ^ 1, P ^ 1);
-    store_bg(P ^ 1, P ^ 1);
     load_a(min(kt + 3, KT - 1), P ^ 1);
-    load_bg(min(kt + 3, KT - 1), P ^ 1);
     __syncthreads();
   };
   for (int kt = 0; kt < KT; kt += 2) {
@@ -632,20 +562,14 @@ gemm16_kernel(GemmArgs p) {
     for (int r = 0; r < 4; ++r) {
       const int gr = m0 + wm * (BMT / 2) + mi * 16 + 4 * kg + r;
       if (gr >= p.M) continue;
-      {
-        if constexpr (EPI == EPI_AFFINE)
-          if (!affine_row(p, gr)) continue;
 #pragma unroll
-        for (int ni = 0; ni < 4; ++ni) {
-          if (!tv[ni]) continue;
-          const size_t o = (size_t)gr * p.ldy + tile[ni] * 16 + row;
-          if constexpr (EPI == EPI_RESID)
-            ((T*)p.y)[o] = st_act<A>(ld_act<A>(rres.v[mi][r][ni]) + rd<A>(acc[mi][ni][r]));
-          else if constexpr (EPI == EPI_AFFINE)
-            ((T*)p.y)[o] = st_act<A>(affine_value<A>(p, acc[mi][ni][r], gr, tile[ni] * 16 + row));
-          else
-            ((T*)p.y)[o] = st_act<A>(acc[mi][ni][r]);
-        }
+      for (int ni = 0; ni < 4; ++ni) {
+        if (!tv[ni]) continue;
+        const size_t o = (size_t)gr * p.ldy + tile[ni] * 16 + row;
+        if constexpr (EPI == EPI_RESID)
+          ((T*)p.y)[o] = st_act<A>(ld_act<A>(rres.v[mi][r][ni]) + rd<A>(acc[mi][ni][r]));
+        else
+          ((T*)p.y)[o] = st_act<A>(acc[mi][ni][r]);
       }
     }
   }
@@ -654,8 +578,8 @@ gemm16_kernel(GemmArgs p) {
 // 16-bit activations with dense 16-bit weights, both operands copied global
 // -> LDS by the direct-to-LDS loads (no register staging): a ring of NS
 // stages of BK2 = 32 k, NS - 1 steps in flight, one barrier per step.  Tile
-// BMT x 128 (BMT 64, 128 or 256), four waves of BMT/2 x 64 (same fragments, same
-// epilogue, same XCD work order as gemm16_kernel).  X stage: BMT rows x 4
+// BMT x 128 (BMT 64, 128 or 256), four waves of BMT/2 x 64 (same fragments and
+// XCD work order as gemm_q8_kernel).  X stage: BMT rows x 4
 // chunks of 8 elements, chunk c of row r at slot r * 4 + (c ^ swz(r)), so
 // that the fragment reads of any 8 consecutive lanes fall in distinct
 // 16-byte bank groups of 128 bytes and those of any 16 in distinct groups of
@@ -922,6 +846,285 @@ gemm_dma_kernel(GemmArgs p) {
   }
 }
 
+// ---------------------------------------------------------------------------
+// Small grids: BM x BN tiles (32 or 64 rows x 32, 64 or 128 columns), four
+// waves in 2 x 2 (BM/2 x BN/2 each), for products whose 64 x 128 tiles would
+// leave most CUs without a work-group.
+//
+// What bounds them is the serial K loop of one work-group, not bytes: the
+// 64 x 128 register-staged tiles took 23 us for K = 3072 at any M up to 2048
+// (32 work-groups on 256 CUs at M = 256), the 33 us of Q8_0 likewise.  A
+// smaller tile has less to copy, read and multiply per k and the ring keeps
+// 30-70 KB of it in flight per work-group: 7.6 us (dense, 32 x 32) and 11.8 us
+// (Q8_0) at M = 256, N = 1024, K = 3072 (try_small has the rule and figures).
+//
+// Both operands (for Q8_0 the quants and the scales too) go global -> LDS by
+// direct-to-LDS loads through a ring of NS stages of KS k, NS - 1 in flight,
+// one barrier per stage.  KS is 64 for dense weights and 128 for Q8_0 (a
+// stage is then a whole number of copies per wave).  X stage: row r is KS / 8
+// chunks of 16 bytes, chunk c at position c ^ swx(r), so that the fragment
+// reads (16 rows, one chunk) fall in distinct banks.  Weight stage: the tiles'
+// fragments as stored; Q8_0 scales: 16 x 2 u32 per tile.  Each output is
+// summed over k in the order of the other tiles by the same MFMAs, so tile
+// kinds give the same bits.
+template <int KS>
+__device__ __forceinline__ int swx(int r) {
+  return KS == 64 ? (r >> 1) & 7 : r & 15;
+}
+
+// Column tile lt (0 .. BN/16 - 1; wave column lt / NI, its fragment lt % NI)
+// of column group cg: EPI_SWIGLU pairs gate tiles (the first half of a wave's
+// fragments) with the matching up tiles.  ok: whether it lies in the product.
+template <int EPI, int BN>
+__device__ __forceinline__ int small_tile(int cg, int ntiles, int lt, bool& ok) {
+  constexpr int NI = BN / 32;
+  if constexpr (EPI == EPI_SWIGLU) {
+    constexpr int G = NI / 2;
+    const int wn = lt / NI, ni = lt % NI;
+    const int base = cg * (BN / 32) + wn * G + ni % G;
+    ok = base < ntiles / 2;
+    return ni < G ? base : base + ntiles / 2;
+  } else {
+    const int t = cg * (BN / 16) + lt;
+    ok = t < ntiles;
+    return t;
+  }
+}
+
+template <int A, int WK, int EPI, int BM, int BN, int KS, int NS>
+__global__ void __launch_bounds__(256) gemm_small_kernel(GemmArgs p) {
+  typedef typename ActT<A>::T T;
+  constexpr bool Q8 = WK == WK_Q8;
+  constexpr int MI = BM / 32, NI = BN / 32, NT = BN / 16;
+  static_assert(EPI != EPI_SWIGLU || NI >= 2, "gate and up tiles in one wave");
+  static_assert(EPI != EPI_ROPE || BN == 128, "one head slot per work-group");
+  constexpr int XB = BM * KS * 2;                 // stage bytes: X rows,
+  constexpr int WB = Q8 ? BN * KS : BN * KS * 2;  // weights,
+  constexpr int SCB = Q8 ? NT * KS : 0;           // scales
+  constexpr int TK = Q8 ? KS / 64 : KS / 32;      // KiB of weights per tile
+  constexpr int SCL = SCB / 64;                   // 16-byte pieces of scales per wave
+  constexpr int SB = XB + WB + SCB;
+  constexpr int NXC = XB / 4096, NWC = WB / 4096; // 1 KiB copies per wave
+  static_assert(XB % 4096 == 0 && WB % 4096 == 0, "whole copies per wave");
+  constexpr int PER = NXC + NWC + (Q8 ? 1 : 0);
+  static_assert((NS - 2) * PER < 64, "vmcnt");
+  constexpr int EPIB = EPI == EPI_ROPE ? BM * 256 : 0;
+  __shared__ __attribute__((aligned(1024))) uint8_t smem[NS * SB > EPIB ? NS * SB : EPIB];
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  const int wm = w >> 1, wn = w & 1, row = lane & 15, kg = lane >> 4;
+  const int K = p.W.in, ntiles = p.W.out / 16;
+  constexpr int CW = EPI == EPI_SWIGLU ? BN / 32 : NT;   // (gate) tiles per column group
+  const int cols = ((EPI == EPI_SWIGLU ? ntiles / 2 : ntiles) + CW - 1) / CW;
+  int mt, cg;
+  tile_of(blockIdx.x, (p.M + BM - 1) / BM, cols, p.map, mt, cg);
+  if (mt * BM >= p.M) return;
+  const int m0 = mt * BM;
+  [[maybe_unused]] RopeRows<EPI == EPI_ROPE ? BM : 16> rrows;
+  if constexpr (EPI == EPI_ROPE) rrows = rope_rows<BM>(p, m0);
+  int tile[NI];
+  bool tv[NI];
+#pragma unroll
+  for (int ni = 0; ni < NI; ++ni) tile[ni] = small_tile<EPI, BN>(cg, ntiles, wn * NI + ni, tv[ni]);
+
+  // The residuals of the elements this lane stores, loaded before the K loop
+  // (rows past M and tiles past the end read clamped addresses).
+  constexpr bool RES = EPI == EPI_RESID || EPI == EPI_AFFINE;
+  [[maybe_unused]] T rres[RES ? MI * 4 * NI : 1];
+  if constexpr (RES) {
+    const T* rp = (const T*)(p.resid ? p.resid : p.y);
+#pragma unroll
+    for (int mi = 0; mi < MI; ++mi)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int gr = min(m0 + wm * (BM / 2) + mi * 16 + 4 * kg + r, p.M - 1);
+#pragma unroll
+        for (int ni = 0; ni < NI; ++ni)
+          rres[(mi * 4 + r) * NI + ni] = rp[(size_t)gr * p.ldy + (tv[ni] ? tile[ni] : 0) * 16 + row];
+      }
+  }
+
+  // This wave's copies per stage.
+  const int wu = __builtin_amdgcn_readfirstlane(w);
+  const uint16_t* xbase = (const uint16_t*)p.x + (size_t)m0 * p.ldx;
+  uint32_t xoff[NXC], woff[NWC], soff = 0;
+#pragma unroll
+  for (int i = 0; i < NXC; ++i) {
+    constexpr int CH = KS / 8;
+    const int piece = (wu * NXC + i) * 64 + lane, r = piece / CH, pos = piece % CH;
+    xoff[i] = (uint32_t)(min(m0 + r, p.M - 1) - m0) * (uint32_t)p.ldx * 2u + (uint32_t)((pos ^ swx<KS>(r)) * 16);
+  }
+#pragma unroll
+  for (int i = 0; i < NWC; ++i) {
+    // copy j is KiB j % TK of column tile j / TK's stage (a KiB is 32 k of
+    // dense weights, 64 k of Q8_0)
+    const int j = wu * NWC + i;
+    bool ok;
+    int tl = small_tile<EPI, BN>(cg, ntiles, j / TK, ok);
+    tl = ok ? tl : ntiles - 1;
+    woff[i] = ((uint32_t)tl * (K / (KS / TK)) + (j % TK)) * 1024u + lane * 16u;
+  }
+  if constexpr (Q8) {
+    const int q = wu * SCL + min(lane, SCL - 1);
+    bool ok;
+    int tl = small_tile<EPI, BN>(cg, ntiles, q / (KS / 16), ok);
+    tl = ok ? tl : ntiles - 1;
+    soff = (uint32_t)tl * K + (q % (KS / 16)) * 16u;
+  }
+  const uint32_t ls = lds_addr(smem);
+  auto issue = [&](int kt, int buf) {
+    const uint32_t b = ls + (uint32_t)(buf * SB);
+#pragma unroll
+    for (int i = 0; i < NXC; ++i)
+      lds_copy16(xbase, xoff[i] + (uint32_t)(kt * KS * 2), b + (uint32_t)((wu * NXC + i) * 1024));
+#pragma unroll
+    for (int i = 0; i < NWC; ++i)
+      lds_copy16(p.W.w, woff[i] + (uint32_t)(kt * TK * 1024), b + (uint32_t)(XB + (wu * NWC + i) * 1024));
+    if constexpr (Q8) {
+      // a quarter of the scales per wave: lanes past its pieces copy nothing
+      if (lane < SCL) lds_copy16(p.W.sc, soff + (uint32_t)(kt * KS), b + (uint32_t)(XB + WB + wu * (SCL * 16)));
+    }
+  };
+
+  f32x4 acc[MI][NI];
+#pragma unroll
+  for (int mi = 0; mi < MI; ++mi)
+#pragma unroll
+    for (int ni = 0; ni < NI; ++ni) acc[mi][ni] = f32x4{0.f, 0.f, 0.f, 0.f};
+  const int KT = K / KS;
+#pragma unroll
+  for (int s0 = 0; s0 < NS - 1; ++s0) issue(min(s0, KT - 1), s0);
+  int slot = 0;   // kt % NS
+  for (int kt = 0; kt < KT; ++kt) {
+    // this stage's copies have landed; the last NS - 2 stages wait for all
+    if (KT - 1 - kt >= NS - 2) wait_vm<(NS - 2) * PER>();
+    else wait_vm<0>();
+    barrier_lds();
+    // refill the slot computed in the previous step
+    if (kt + NS - 1 < KT) issue(kt + NS - 1, slot == 0 ? NS - 1 : slot - 1);
+    const uint16_t* a = (const uint16_t*)(smem + slot * SB);
+    const uint8_t* bb = smem + slot * SB + XB;
+    if constexpr (Q8) {
+      const uint32_t* sc = (const uint32_t*)(bb + WB);
+#pragma unroll
+      for (int c = 0; c < TK; ++c) {
+        u32x4 fa[MI][2];
+#pragma unroll
+        for (int mi = 0; mi < MI; ++mi)
+#pragma unroll
+          for (int ks = 0; ks < 2; ++ks) {
+            const int r = wm * (BM / 2) + mi * 16 + row;
+            fa[mi][ks] = *(const u32x4*)&a[r * KS + (((8 * c + 4 * ks + kg) ^ swx<KS>(r)) << 3)];
+          }
+#pragma unroll
+        for (int ni = 0; ni < NI; ++ni) {
+          const int lt = wn * NI + ni;
+          const u32x4 cb = *(const u32x4*)(bb + (lt * TK + c) * 1024 + lane * 16);
+          const uint32_t cs = sc[(lt * TK + c) * 16 + row];
+          const u32x4 b0 = q8_to_f16x8(cb[0], cb[1]);
+          const u32x4 b1 = q8_to_f16x8(cb[2], cb[3]);
+          const float d0 = f16_to_f32((uint16_t)(cs & 0xffffu));
+          const float d1 = f16_to_f32((uint16_t)(cs >> 16));
+          const f32x4 z = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+          for (int mi = 0; mi < MI; ++mi) {
+            const f32x4 t0 = mfma16<ACT_F16>(fa[mi][0], b0, z);
+            const f32x4 t1 = mfma16<ACT_F16>(fa[mi][1], b1, z);
+            acc[mi][ni] += d0 * t0;
+            acc[mi][ni] += d1 * t1;
+          }
+        }
+      }
+    } else {
+#pragma unroll
+      for (int ks = 0; ks < TK; ++ks) {
+        u32x4 fb[NI];
+#pragma unroll
+        for (int ni = 0; ni < NI; ++ni)
+          fb[ni] = *(const u32x4*)(bb + ((wn * NI + ni) * TK + ks) * 1024 + lane * 16);
+#pragma unroll
+        for (int mi = 0; mi < MI; ++mi) {
+          const int r = wm * (BM / 2) + mi * 16 + row;
+          const u32x4 fa = *(const u32x4*)&a[r * KS + (((4 * ks + kg) ^ swx<KS>(r)) << 3)];
+#pragma unroll
+          for (int ni = 0; ni < NI; ++ni) acc[mi][ni] = mfma16<A>(fa, fb[ni], acc[mi][ni]);
+        }
+      }
+    }
+    slot = slot + 1 == NS ? 0 : slot + 1;
+  }
+
+  if constexpr (EPI == EPI_ROPE) {
+    rope_epilogue<A, BM, MI>(p, acc, (T*)smem, m0, cg, rrows);
+    return;
+  }
+  if constexpr (EPI == EPI_SWIGLU) {
+    constexpr int G = NI / 2;
+#pragma unroll
+    for (int mi = 0; mi < MI; ++mi)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int gr = m0 + wm * (BM / 2) + mi * 16 + 4 * kg + r;
+#pragma unroll
+        for (int ni = 0; ni < G; ++ni) {
+          const float gg = rd<A>(acc[mi][ni][r]), u = rd<A>(acc[mi][ni + G][r]);
+          const float o = rd<A>(gg / (1.0f + __expf(-gg))) * u;
+          if (gr < p.M && tv[ni]) ((T*)p.y)[(size_t)gr * p.ldy + tile[ni] * 16 + row] = st_act<A>(o);
+        }
+      }
+    return;
+  }
+  if constexpr (EPI == EPI_AFFINE) {
+    constexpr int N = MI * 4 * NI;
+    float v[N], sc[N], bs[N];
+    T tb[N];
+#pragma unroll
+    for (int ni = 0; ni < NI; ++ni) {
+      const int col = (tv[ni] ? tile[ni] : 0) * 16 + row;
+      const float b = p.aff.bias ? ld_act<A>(((const T*)p.aff.bias)[col]) : 0.f;
+      const float s1 = col < p.aff.scale_cols ? p.aff.scale : 1.f;
+#pragma unroll
+      for (int mi = 0; mi < MI; ++mi)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const int e = (mi * 4 + r) * NI + ni;
+          const int gr = min(m0 + wm * (BM / 2) + mi * 16 + 4 * kg + r, p.M - 1);
+          v[e] = acc[mi][ni][r];
+          bs[e] = b;
+          sc[e] = s1;
+          tb[e] = p.aff.table ? ((const T*)p.aff.table)[(size_t)min(gr % p.aff.period, p.aff.valid - 1) * p.W.out + col] : (T)0;
+        }
+    }
+    affine_block<A, N, false>(p, v, sc, bs, rres, tb);
+#pragma unroll
+    for (int mi = 0; mi < MI; ++mi)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int gr = m0 + wm * (BM / 2) + mi * 16 + 4 * kg + r;
+        if (gr >= p.M || !affine_row(p, gr)) continue;
+#pragma unroll
+        for (int ni = 0; ni < NI; ++ni)
+          if (tv[ni]) ((T*)p.y)[(size_t)gr * p.ldy + tile[ni] * 16 + row] = st_act<A>(v[(mi * 4 + r) * NI + ni]);
+      }
+    return;
+  }
+#pragma unroll
+  for (int mi = 0; mi < MI; ++mi)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int gr = m0 + wm * (BM / 2) + mi * 16 + 4 * kg + r;
+      if (gr >= p.M) continue;
+#pragma unroll
+      for (int ni = 0; ni < NI; ++ni) {
+        if (!tv[ni]) continue;
+        const size_t o = (size_t)gr * p.ldy + tile[ni] * 16 + row;
+        if constexpr (EPI == EPI_RESID)
+          ((T*)p.y)[o] = st_act<A>(ld_act<A>(rres[(mi * 4 + r) * NI + ni]) + rd<A>(acc[mi][ni][r]));
+        else
+          ((T*)p.y)[o] = st_act<A>(acc[mi][ni][r]);
+      }
+    }
+}
+
 // f32 activations / weights on v_mfma_f32_16x16x4f32; same tiling, K chunks of 16.
 template <int EPI>
 __global__ void __launch_bounds__(256) gemm32_kernel(GemmArgs p) {
@@ -1009,29 +1212,23 @@ __global__ void __launch_bounds__(256) gemm32_kernel(GemmArgs p) {
   }
 }
 
-// Tile of the 16-bit dense kernels (512 work-groups = two per CU), chosen
-// from bf16 sweeps over the prefill shapes and row counts:
-// - 256 rows (DMA) where 256-row tiles fill at least 7/8 of the slots and do
-//   not end in a last round of fewer than 128 work-groups (qkv M = 3584 36.5
-//   against 38.9 us, M = 4096 39.2 against 42.4; gate|up M = 2560 38.0
-//   against 41.4, M = 4096 59.8 against 62.9, but M = 3072, 576 tiles, 56.2
-//   against 51.9);
-// - 128 rows (DMA) where their grid fills the slots, and for wide outputs
-//   (16 or more column groups) also below that (qkv M = 1328 19.5 against
-//   22.3 us for 64-row tiles, M = 1560 20.9 against 27.6);
-// - narrow outputs (O and down, N = 1024) otherwise take 64-row tiles: the
-//   register-staged kernel up to one tile per CU, the DMA kernel above
-//   (O M = 2048 23.3 against 25.3 us; M = 2455 28.4 against 32.3, M = 4096
-//   31.7 against 34.7; down M = 2455 37.5 against 43.0, M = 4096 42.0
-//   against 46.0).
-enum GemmTile { TILE64 = 0, TILE64_DMA = 1, TILE128 = 2, TILE256 = 3 };
+// Tile of the 16-bit dense products past the small grids (512 work-groups =
+// two per CU), chosen from bf16 sweeps over the prefill shapes and row counts:
+// - 256 rows where 256-row tiles fill at least 7/8 of the slots and do not end
+//   in a last round of fewer than 128 work-groups (qkv M = 3584 36.5 against
+//   38.9 us, M = 4096 39.2 against 42.4; gate|up M = 2560 38.0 against 41.4,
+//   M = 4096 59.8 against 62.9, but M = 3072, 576 tiles, 56.2 against 51.9);
+// - 128 rows where their grid fills the slots, and for wide outputs (16 or more
+//   column groups) also below that (qkv M = 1328 19.5 against 22.3 us for
+//   64-row tiles, M = 1560 20.9 against 27.6);
+// - narrow outputs otherwise take 64 rows.
+enum GemmTile { TILE64, TILE128, TILE256 };
 GemmTile gemm_tile(int M, int col_groups) {
-  const int tiles64 = (M + 63) / 64 * col_groups;
   const int tiles128 = (M + 127) / 128 * col_groups;
   const int tiles256 = (M + 255) / 256 * col_groups;
   if (tiles256 >= 448 && (tiles256 % 512 == 0 || tiles256 % 512 >= 128)) return TILE256;
   if (tiles128 >= 512 || col_groups >= 16) return TILE128;
-  return tiles64 > 256 ? TILE64_DMA : TILE64;
+  return TILE64;
 }
 
 // 16-byte output, bias, residual and table accesses for the staged
@@ -1059,7 +1256,7 @@ hipError_t launch_dma(int epi, dim3 grid, const GemmArgs& a, hipStream_t s) {
       else hipLaunchKernelGGL((gemm_dma_kernel<A, EPI_ROPE, BMT, NS>), grid, dim3(256), 0, s, a);
       break;
     case EPI_AFFINE:
-      if (!staged_ok(a)) return hipErrorInvalidValue;  // dispatch routes these to the 64-row tiles
+      if (!staged_ok(a)) return hipErrorInvalidValue;  // try_small takes these
       hipLaunchKernelGGL((gemm_dma_kernel<A, EPI_AFFINE, BMT, NS>), grid, dim3(256), 0, s, a);
       break;
     default: return hipErrorInvalidValue;
@@ -1067,29 +1264,15 @@ hipError_t launch_dma(int epi, dim3 grid, const GemmArgs& a, hipStream_t s) {
   return hipGetLastError();
 }
 
-template <int A, int WK, int BMT, bool LB>
-hipError_t launch16_lb(int epi, dim3 grid, const GemmArgs& a, hipStream_t s) {
+hipError_t launch_q8(int epi, dim3 grid, const GemmArgs& a, hipStream_t s) {
   switch (epi) {
-    case EPI_STORE: hipLaunchKernelGGL((gemm16_kernel<A, WK, EPI_STORE, BMT, LB>), grid, dim3(256), 0, s, a); break;
-    case EPI_RESID: hipLaunchKernelGGL((gemm16_kernel<A, WK, EPI_RESID, BMT, LB>), grid, dim3(256), 0, s, a); break;
-    case EPI_SWIGLU: hipLaunchKernelGGL((gemm16_kernel<A, WK, EPI_SWIGLU, BMT, LB>), grid, dim3(256), 0, s, a); break;
-    case EPI_ROPE: hipLaunchKernelGGL((gemm16_kernel<A, WK, EPI_ROPE, BMT, LB>), grid, dim3(256), 0, s, a); break;
-    case EPI_AFFINE:
-      if constexpr (WK == WK_Q8) return hipErrorInvalidValue;  // the audio path is dense
-      else hipLaunchKernelGGL((gemm16_kernel<A, WK, EPI_AFFINE, BMT, LB>), grid, dim3(256), 0, s, a);
-      break;
-    default: return hipErrorInvalidValue;
+    case EPI_STORE: hipLaunchKernelGGL((gemm_q8_kernel<EPI_STORE>), grid, dim3(256), 0, s, a); break;
+    case EPI_RESID: hipLaunchKernelGGL((gemm_q8_kernel<EPI_RESID>), grid, dim3(256), 0, s, a); break;
+    case EPI_SWIGLU: hipLaunchKernelGGL((gemm_q8_kernel<EPI_SWIGLU>), grid, dim3(256), 0, s, a); break;
+    case EPI_ROPE: hipLaunchKernelGGL((gemm_q8_kernel<EPI_ROPE>), grid, dim3(256), 0, s, a); break;
+    default: return hipErrorInvalidValue;  // the audio path is dense
   }
   return hipGetLastError();
-}
-
-// Dense weights of 64-row tiles go through LDS; 128-row tiles read them from
-// global memory (measured: staging made the 64-row tiles ~4% faster and the
-// 128-row tiles ~8% slower, whose LDS reads then outlast the MFMAs).
-template <int A, int WK, int BMT>
-hipError_t launch16(int epi, dim3 grid, const GemmArgs& a, hipStream_t s) {
-  if constexpr (WK == WK_DENSE && BMT == 64) return launch16_lb<A, WK, BMT, true>(epi, grid, a, s);
-  return launch16_lb<A, WK, BMT, false>(epi, grid, a, s);
 }
 
 // XCD rows a (1, 2, 4 or 8; the XCD grid is a x 8/a) for an M x N x K
@@ -1109,6 +1292,84 @@ int xcd_rows(const GemmArgs& p, int cols, int bm) {
   return best;
 }
 
+template <int A, int WK, int BM, int BN, int KS, int NS>
+hipError_t launch_small(int epi, const GemmArgs& a, hipStream_t s) {
+  const int ntiles = a.W.out / 16;
+  const int cw = epi == EPI_SWIGLU ? BN / 32 : BN / 16;
+  const int cols = ((epi == EPI_SWIGLU ? ntiles / 2 : ntiles) + cw - 1) / cw;
+  GemmArgs g = a;
+  g.map = xcd_rows(a, cols, BM);
+  const int mtiles = (a.M + BM - 1) / BM, Ma = (mtiles + g.map - 1) / g.map;
+  const dim3 grid(8 * Ma * (cols / (8 / g.map)));
+#define SMALL(E) hipLaunchKernelGGL((gemm_small_kernel<A, WK, E, BM, BN, KS, NS>), grid, dim3(256), 0, s, g)
+  switch (epi) {
+    case EPI_ROPE:
+      if constexpr (BN == 128) { SMALL(EPI_ROPE); break; }
+      return hipErrorInvalidValue;
+    case EPI_SWIGLU:
+      if constexpr (BN == 64) { SMALL(EPI_SWIGLU); break; }
+      return hipErrorInvalidValue;
+    case EPI_AFFINE:   // the audio path is dense
+      if constexpr (BN < 128 && WK != WK_Q8) { SMALL(EPI_AFFINE); break; }
+      return hipErrorInvalidValue;
+    case EPI_STORE:
+      if constexpr (BN < 128) { SMALL(EPI_STORE); break; }
+      return hipErrorInvalidValue;
+    case EPI_RESID:
+      if constexpr (BN < 128) { SMALL(EPI_RESID); break; }
+      return hipErrorInvalidValue;
+    default: return hipErrorInvalidValue;
+  }
+#undef SMALL
+  return hipGetLastError();
+}
+
+// Tiles of the small grids: the smallest tile whose grid does not exceed
+// `most` work-groups (one or two per CU), so that every CU has one while each
+// work-group's serial K loop stays short; past all of them the tiles above.
+// us per product (this rule's tile | the 64- and 128-row tiles above):
+//   dense N = 1024, K = 3072: M = 100 7.2 | 22.4, 256 7.6 | 22.8, 450 10.6 |
+//   22.7, 1024 14.6 | 23.0, 2048 20.7 | 24.0, 4096 31.1 | 34.6;
+//   dense N = 4096, K = 1024: M = 24 4.5 | 12.3, 100 5.1 | 12.7, 256 6.9 |
+//   12.9, 450 9.4 | 13.3, 1024 13.7 | 14.7, but 1501 (768 work-groups) 21.4 |
+//   19.1;
+//   Q8_0 N = 1024, K = 3072: M = 100 11.4 | 33.1, 256 11.8 | 33.2, 1024 20.7 |
+//   34.4, 2048 33.8 | 35.1, but 3002 52.0 | 48.0;
+//   Q8_0 N = 4096, K = 1024: M = 24 5.0 | 13.7, 256 8.9 | 13.7, 450 13.8 |
+//   14.4, but 700 21.5 | 19.4.
+// EPI_ROPE needs 128 columns (a head slot) and EPI_SWIGLU 64 (a gate and an up
+// tile in each wave).  false: no tile applies.
+template <int A, int WK>
+bool try_small(int epi, const GemmArgs& a, hipStream_t s, hipError_t* e) {
+  const int ntiles = epi == EPI_SWIGLU ? a.W.out / 32 : a.W.out / 16, K = a.W.in;
+  const bool n32 = epi != EPI_ROPE && epi != EPI_SWIGLU, n64 = epi != EPI_ROPE;
+  // grid of BM x BN tiles (a gate and an up tile count as one)
+  auto fits = [&](int bm, int bn, int ks, int most) {
+    const int cw = epi == EPI_SWIGLU ? bn / 32 : bn / 16;
+    return K % ks == 0 && (int64_t)((a.M + bm - 1) / bm) * ((ntiles + cw - 1) / cw) <= most;
+  };
+  if constexpr (WK == WK_Q8) {
+    if (n32 && fits(32, 32, 256, 256)) *e = launch_small<A, WK, 32, 32, 256, 3>(epi, a, s);
+    else if (n32 && fits(64, 32, 128, 512)) *e = launch_small<A, WK, 64, 32, 128, 3>(epi, a, s);
+    else if (n64 && fits(64, 64, 128, 512)) *e = launch_small<A, WK, 64, 64, 128, 3>(epi, a, s);
+    else if (!n64 && fits(32, 128, 128, 256)) *e = launch_small<A, WK, 32, 128, 128, 3>(epi, a, s);
+    else return false;
+  } else {
+    // the direct-to-LDS tiles' affine epilogue moves 16 bytes at a time; an
+    // output, residual, bias or table that does not allow it stays here
+    const bool stay = epi == EPI_AFFINE && !staged_ok(a);
+    if (n32 && fits(32, 32, 128, 256)) *e = launch_small<A, WK, 32, 32, 128, 4>(epi, a, s);
+    else if (n64 && fits(32, 64, 128, 256)) *e = launch_small<A, WK, 32, 64, 128, 3>(epi, a, s);
+    else if (n64 && fits(64, 64, 128, 256)) *e = launch_small<A, WK, 64, 64, 128, 3>(epi, a, s);
+    else if (n64 && fits(64, 64, 64, 512)) *e = launch_small<A, WK, 64, 64, 64, 4>(epi, a, s);
+    else if (n64 && (stay || fits(128, 64, 64, 512))) *e = launch_small<A, WK, 128, 64, 64, 3>(epi, a, s);
+    else if (!n64 && fits(32, 128, 64, 256)) *e = launch_small<A, WK, 32, 128, 64, 4>(epi, a, s);
+    else if (!n64 && fits(64, 128, 64, 512)) *e = launch_small<A, WK, 64, 128, 64, 3>(epi, a, s);
+    else return false;
+  }
+  return true;
+}
+
 template <int A, int WK>
 hipError_t dispatch(int epi, const GemmArgs& a, hipStream_t s) {
   const int ntiles = a.W.out / 16;
@@ -1124,11 +1385,11 @@ hipError_t dispatch(int epi, const GemmArgs& a, hipStream_t s) {
     }
     return hipGetLastError();
   } else {
+    {
+      hipError_t e = hipSuccess;
+      if (try_small<A, WK>(epi, a, s, &e)) return e;
+    }
     GemmTile tt = WK == WK_Q8 ? TILE64 : gemm_tile(a.M, cols);
-    // the direct-to-LDS tiles' affine epilogue moves 16 bytes at a time; an
-    // output, residual, bias or table that does not allow it takes the
-    // register-staged tiles (element by element)
-    if (epi == EPI_AFFINE && tt != TILE64 && !staged_ok(a)) tt = TILE64;
     // the fused q/k norm + RoPE epilogue stages at most 128 rows (a 256-row
     // tile would spill), and the residuals a 256-row tile would prefetch do
     // not fit its registers: 128-row tiles instead
@@ -1138,15 +1399,12 @@ hipError_t dispatch(int epi, const GemmArgs& a, hipStream_t s) {
     g.map = xcd_rows(a, cols, bm);
     const int mtiles = (a.M + bm - 1) / bm, Ma = (mtiles + g.map - 1) / g.map;
     const dim3 grid(8 * Ma * (cols / (8 / g.map)));
-    // Q8_0 tiles scale each block's product in f32 on the VALU, so their
-    // accumulators live in VGPRs: only the 64-row tile fits without spills.
-    if (tt == TILE64) return launch16<A, WK, 64>(epi, grid, g, s);
-    if constexpr (WK != WK_Q8) {
+    if constexpr (WK == WK_Q8) return launch_q8(epi, grid, g, s);
+    else {
       if (tt == TILE256) return launch_dma<A, 256, 3>(epi, grid, g, s);
       if (tt == TILE128) return launch_dma<A, 128, 4>(epi, grid, g, s);
       return launch_dma<A, 64, 4>(epi, grid, g, s);
     }
-    return hipErrorInvalidValue;
   }
 }
 

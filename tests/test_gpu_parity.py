@@ -136,10 +136,9 @@ def test_linear_projections(fmd, orc, prec, rows):
                                        ("int8", 130), ("int8", 2100)])
 def test_linear_projections_gemm_tiles(fmd, orc, prec, rows):
     """Prefill GEMM at full widths: ragged last row tiles, the padded XCD
-    blocks of every projection shape, and for bf16 each tile kind: 130 rows
-    64-row register-staged (O, down) and 128-row (qkv, gate|up) tiles, 2100
-    rows 64-row direct-to-LDS (O, down) and 128-row tiles, 4000 rows 256-row
-    (qkv, gate|up) tiles."""
+    blocks of every projection shape, and several tile kinds: 130 rows
+    small-grid tiles, for bf16 2100 rows 128 x 64 (O, down) and 128-row tiles,
+    4000 rows 256-row (qkv, gate|up) tiles."""
     _announce(f"gemm tiles {prec} rows={rows}")
     cfg = small_cfg(fmd, layers=1, vocab=256)
     gpu, ref, w = build_pair(fmd, orc, cfg, prec, seed=33, max_len=64)
@@ -163,6 +162,48 @@ def test_linear_projections_gemm_tiles(fmd, orc, prec, rows):
         Wd = orc.dequantize_q8_0(orc.quantize_q8_0(W), *W.shape) if prec == "int8" else W
         tol = ulp * np.abs(want) + 1e-6 * (np.abs(x) @ np.abs(Wd).T) + 1e-7
         assert np.all(np.abs(got - want) <= tol), (proj, np.max(np.abs(got - want) - tol))
+
+
+@pytest.mark.parametrize("prec", ["f16", "bf16", "int8"])
+def test_linear_tile_kinds_give_the_same_bits(fmd, prec):
+    """Every tile kind sums an output over k in the same order with the same
+    MFMAs: the first m rows of a product are the same bits for every m, through
+    the row counts where the tile changes at each width (and their edges), up
+    to one past the small grids."""
+    _announce(f"gemm tile kinds {prec}")
+    cfg = small_cfg(fmd, layers=1, vocab=256)
+    gpu = fmd.Qwen3(cfg, prec, max_len=64).load(fmd.synthetic_weights(cfg, seed=35))
+    dt = torch.bfloat16 if prec == "bf16" else torch.float16
+    for proj, (k, n) in {0: (1024, 4096), 1: (2048, 1024), 2: (1024, 6144), 3: (3072, 1024)}.items():
+        x = torch.randn((4300, k), generator=torch.Generator().manual_seed(proj)).to(dt).cuda()
+        full = torch.empty((4300, n), dtype=dt, device="cuda")
+        torch.cuda.synchronize()
+        gpu.op_linear(0, proj, x.data_ptr(), 4300, full.data_ptr())
+        for m in (17, 31, 33, 64, 65, 129, 255, 257, 511, 513, 700, 1023, 1025, 2049, 4095, 4097):
+            y = torch.empty((m, n), dtype=dt, device="cuda")
+            gpu.op_linear(0, proj, x.data_ptr(), m, y.data_ptr())
+            torch.cuda.synchronize()
+            assert torch.equal(y, full[:m]), (proj, m)
+
+
+@pytest.mark.parametrize("prec,n", [("int8", 20), ("int8", 225), ("int8", 450), ("f16", 65),
+                                    ("bf16", 257), ("bf16", 700)])
+def test_prefill_small_grids_full_width(fmd, orc, prec, n):
+    """One prompt in one chunk at full layer widths: the small-grid tiles with
+    the residual, SwiGLU and RoPE epilogues, against the oracle."""
+    _announce(f"prefill small grids {prec} n={n}")
+    cfg = small_cfg(fmd, layers=1, vocab=512)
+    gpu, ref, _ = build_pair(fmd, orc, cfg, prec, seed=36, max_len=1024)
+    rng = np.random.default_rng(n)
+    emb, pad = ref.padded_embeds([rng.integers(0, cfg.vocab_size, n).tolist()])
+    gkv, rkv = gpu.new_caches(1, n + 4), ref.new_kv(1, n + 4)
+    got = gpu.prefill(orc.to_storage(emb, OPREC[prec]), gkv, pad, chunk=1024)
+    want = ref.prefill(rkv, emb, pad, block=256)
+    assert np.max(np.abs(got - want)) < TOL[prec]
+    for which in (0, 1):
+        g, r = storage_to_f32(gkv.read(0, which), prec), rkv.read(0, which)
+        ulp = np.exp2(np.floor(np.log2(np.maximum(np.abs(r), 2.0 ** -14))) - (7 if prec == "bf16" else 10))
+        assert np.all(np.abs(g - r) <= np.maximum(TOL[prec], ulp * 1.0001)), which
 
 
 # --------------------------------------------------------------------------
