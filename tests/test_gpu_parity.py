@@ -206,6 +206,29 @@ def test_prefill_small_grids_full_width(fmd, orc, prec, n):
         assert np.all(np.abs(g - r) <= np.maximum(TOL[prec], ulp * 1.0001)), which
 
 
+@pytest.mark.parametrize("lens,chunk", [((70, 1, 64), 1024), ((900, 130, 65), 256), ((1500,), 512)])
+def test_prefill_f16_running_reference(fmd, orc, lens, chunk):
+    """f16 prefill attention keeps a running reference per row: q and k norm
+    gains of 3 give scores of standard deviation 9, so that later key blocks
+    and items exceed a row's reference by more than the 2^8 it may lag, in
+    one-item tiles (short prompts), split tiles and the combine."""
+    _announce(f"prefill f16 running reference {lens} chunk={chunk}")
+    cfg = tiny_cfg(fmd, layers=1)
+    w = fmd.synthetic_weights(cfg, seed=37)
+    for n in ("q_norm", "k_norm"):
+        w[f"model.language_model.layers.0.self_attn.{n}.weight"][:] = 3.0
+    gpu, ref, _ = build_pair(fmd, orc, cfg, "f16", max_len=2048, weights=w)
+    rng = np.random.default_rng(sum(lens))
+    emb, pad = ref.padded_embeds([rng.integers(0, cfg.vocab_size, n).tolist() for n in lens])
+    gkv, rkv = gpu.new_caches(len(lens), max(lens) + 4), ref.new_kv(len(lens), max(lens) + 4)
+    got = gpu.prefill(orc.to_storage(emb, OPREC["f16"]), gkv, pad, chunk=chunk)
+    want = ref.prefill(rkv, emb, pad, block=256)
+    assert np.all(np.isfinite(got))
+    d = float(np.max(np.abs(got - want)))
+    print(f"[gap] running reference {lens}: max {d:.4g}", flush=True)
+    assert d < TOL["f16"], d
+
+
 # --------------------------------------------------------------------------
 # decode step over a synthetic padded context (configs 2 / 3 style)
 # --------------------------------------------------------------------------
