@@ -634,15 +634,16 @@ struct EpochTag {
   __device__ __forceinline__ uint32_t make(uint32_t e) const { return e; }
   __device__ __forceinline__ uint32_t get() const { return make(load()); }
 };
-__device__ __forceinline__ void fail_sync(uint32_t* sync, uint32_t code) {
+__device__ __forceinline__ void fail_sync(uint32_t* sync, uint32_t* host_err, uint32_t code) {
   __hip_atomic_store(sync + 2, code, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  if (host_err) __hip_atomic_store(host_err, code, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 // A wait gives up past `limit` polls (recording `code`), or as soon as some
 // other wait of the launch has given up (every 64 polls it checks), so a
 // failing launch drains after about one limit's worth of polls.
-__device__ __forceinline__ bool give_up(uint32_t* sync, int spins, int limit, uint32_t code) {
+__device__ __forceinline__ bool give_up(uint32_t* sync, uint32_t* host_err, int spins, int limit, uint32_t code) {
   if (spins >= limit) {
-    fail_sync(sync, code);
+    fail_sync(sync, host_err, code);
     return true;
   }
   return (spins & 63) == 63 &&
@@ -718,7 +719,7 @@ __device__ __forceinline__ void fused_score(const AttnDecodeArgs& p, int split, 
 #pragma unroll
           for (int t = 0; t < 4; ++t) ok = ok && (r >= nw || word_ok(wv[r][t], Ew));
         if (__all(ok)) break;
-        if (give_up(p.sync, spins, p.spin_limit, 5)) break;
+        if (give_up(p.sync, p.host_err, spins, p.spin_limit, 5)) break;
         __builtin_amdgcn_s_sleep(2);
         fetch();
       }
@@ -986,7 +987,7 @@ __device__ __forceinline__ void fused_value(const AttnDecodeArgs& p, int split, 
 #pragma unroll
         for (int t = 0; t < 4; ++t) ok = ok && word_ok(vw[t], E);
         if (ok) break;
-        if (give_up(p.sync, spins, p.spin_limit, 6)) break;
+        if (give_up(p.sync, p.host_err, spins, p.spin_limit, 6)) break;
         __builtin_amdgcn_s_sleep(2);
 #pragma unroll
         for (int t = 0; t < 4; ++t) vw[t] = get_word(p.xqkv + (size_t)b * (p.ldqkv / 2) + vcol / 2 + t);
@@ -995,7 +996,7 @@ __device__ __forceinline__ void fused_value(const AttnDecodeArgs& p, int split, 
     vnew.v = u32x4{(uint32_t)vw[0], (uint32_t)vw[1], (uint32_t)vw[2], (uint32_t)vw[3]};
   }
   for (int spins = 0; !polled(); ++spins) {
-    if (give_up(p.sync, spins, p.spin_limit, 1)) break;
+    if (give_up(p.sync, p.host_err, spins, p.spin_limit, 1)) break;
     __builtin_amdgcn_s_sleep(2);
     poll();
   }
@@ -1131,7 +1132,7 @@ __device__ __forceinline__ void fused_value(const AttnDecodeArgs& p, int split, 
           vj[u] = word_f32(x);
         }
         if (ok) break;
-        if (give_up(p.sync, spins, p.spin_limit, 2)) break;
+        if (give_up(p.sync, p.host_err, spins, p.spin_limit, 2)) break;
         __builtin_amdgcn_s_sleep(2);
       }
 #pragma unroll

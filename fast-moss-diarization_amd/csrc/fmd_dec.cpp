@@ -511,6 +511,8 @@ extern "C" int fmd_kv_destroy(fmd_kv* kv) {
   return 0;
 }
 
+// The length is the host's (kv->len); a call whose kernels read it from
+// kv->state writes it there first (decode_setup, or this before a greedy loop).
 int kv_sync_state(fmd_kv* kv) {
   // state[0] = length (write cursor), [1] = greedy step, [2] = rows done.
   int32_t st[4] = {kv->len, 0, 0, 0};
@@ -523,8 +525,6 @@ extern "C" int fmd_kv_len(const fmd_kv* kv) { return kv ? kv->len : -1; }
 extern "C" int fmd_kv_truncate(fmd_kv* kv, int len) {
   if (!kv) return fmd_fail(FMD_ERR_ARG, "null handle");
   kv->len = std::min(kv->len, std::max(len, 0));
-  CHK(kv_sync_state(kv));
-  HIPCHK(hipStreamSynchronize(kv->dec->stream));
   return 0;
 }
 
@@ -532,8 +532,6 @@ extern "C" int fmd_kv_set_len(fmd_kv* kv, int len) {
   if (!kv) return fmd_fail(FMD_ERR_ARG, "null handle");
   if (len < 0 || len > kv->cap) return fmd_fail(FMD_ERR_ARG, "length outside the capacity");
   kv->len = len;
-  CHK(kv_sync_state(kv));
-  HIPCHK(hipStreamSynchronize(kv->dec->stream));
   return 0;
 }
 

@@ -78,7 +78,7 @@ struct fmd_dec {
   bool embed_set = false, norm_set = false, lm_head_set = false, lm_head_explicit = false;
   DevBuf staging, staging2;
   Workspace ws;
-  int32_t* host_mirror = nullptr;  // host-mapped copy of the greedy state
+  int32_t* host_mirror = nullptr;  // host-mapped copy of the greedy state and the attention error code
   void* host_stage = nullptr;      // pinned host staging of prefill chunk tables
   size_t host_stage_n = 0;
   // what fmd_op_attention_decode last uploaded (repeated calls skip the copies)

@@ -131,6 +131,7 @@ struct AttnDecodeArgs {
   int xsc_stride;         // >= max_splits * split / 2
   uint64_t* xnew;         // (B*nkv, REP) the new token's score, f32
   int spin_limit;         // polls before a wait gives up and records an error
+  uint32_t* host_err;     // host-mapped copy of the error code (NULL: sync[2] only)
   int count_units;        // the launch advances its own epoch once its last unit is
                           // combined (0: the kernel after it advances the epoch)
   // With nq > 0 the launch also computes qkv itself (ldqkv = nq * 16 columns):
@@ -226,6 +227,16 @@ hipError_t launch_rope_store(int act, const RopeArgs& a, hipStream_t s);
 hipError_t launch_attn_decode(int act, const AttnDecodeArgs& a, hipStream_t s);
 hipError_t launch_attn_prefill(int act, int rep, const AttnPrefillArgs& a, hipStream_t s);
 hipError_t launch_greedy(int act, const GreedyArgs& a, hipStream_t s);
+// What a decode call uploads, as kernel arguments instead of host-to-device
+// copies: the write position and the pads to the device words `state` (4) and
+// `pad`; with a table, row ids[b] of it to row b of x.
+struct DecodeSetup {
+  int32_t pad[16];
+  uint32_t ids[16];
+  int32_t len, batch;   // batch <= 16
+};
+hipError_t launch_decode_setup(const DecodeSetup& a, int32_t* state, int32_t* pad, const void* table,
+                               int row_bytes, void* x, hipStream_t s);
 hipError_t launch_embed(int act, const uint32_t* ids, int n, const void* table, int hidden,
                         void* out, hipStream_t s);
 hipError_t launch_gather_rows(int act, const void* src, int ld_src, const int32_t* rows, int n,

@@ -38,6 +38,9 @@ int attn_prefill_tile_rows(int rep);
 namespace {
 
 constexpr int kMaxDecodeRows = 16;
+// Words of fmd_dec::host_mirror: [0, 3) the greedy state, then the error code
+// of the single-launch attention.
+constexpr int kMirrorState = 3, kMirrorErr = 8;
 
 float act_scale(const fmd_dec* d) {
   // scores * scale runs in the activation dtype (qwen3.rs:243).
@@ -56,13 +59,16 @@ int xsc_stride(const AttnDecodePlan& pl) { return pl.max_splits * pl.split / 2 +
 // work-groups of a unit did not all run within the spin limit, e.g. while
 // another kernel held the device); read after the streams are synchronised.
 int check_attn_sync(fmd_dec* d) {
+  // the kernels copy the code to host-mapped memory, so that a call that went
+  // well reads one host word instead of copying from the device
   DecodeLane& ln = d->ws.dec;
-  if (!ln.xsync.p) return 0;
-  uint32_t code = 0;
-  HIPCHK(hipMemcpy(&code, ln.xsync.as<uint32_t>() + 2, 4, hipMemcpyDeviceToHost));
+  if (!ln.xsync.p || !d->host_mirror) return 0;
+  volatile int32_t* word = d->host_mirror + kMirrorErr;
+  const uint32_t code = (uint32_t)*word;
   if (!code) return 0;
   const uint32_t zero = 0;
   HIPCHK(hipMemcpy(ln.xsync.as<uint32_t>() + 2, &zero, 4, hipMemcpyHostToDevice));
+  *word = 0;
   return fmd_fail(FMD_ERR_HIP, "decode attention: work-groups of one (row, KV head) did not meet "
                                "within the spin limit (code " + std::to_string(code) + ")");
 }
@@ -106,6 +112,7 @@ AttnDecodeArgs attn_args(fmd_dec* d, fmd_kv* kv, int layer, int B, const void* q
   a.xsc_stride = xsc_stride(sg);
   a.xnew = ln.xnew.as<uint64_t>();
   a.spin_limit = d->spin_limit;
+  a.host_err = (uint32_t*)(d->host_mirror ? d->host_mirror + kMirrorErr : nullptr);
   a.count_units = 1;
   return a;
 }
@@ -193,14 +200,14 @@ GemvArgs gemv_args(const void* x, int ldx, const void* norm, float eps, const Li
 // qwen3.rs:322-339): the qkv projection (inside the attention launch for
 // 16-bit activations), the attention with the q/k norm, RoPE and cache
 // append, then O + residual, RMSNorm + gate|up + SwiGLU, down + residual.
-// The residual stream is ws.x; the write position is kv->state[0].
-int decode_layer(fmd_dec* d, fmd_kv* kv, int l, int B, const int32_t* pad_dev,
+// x (B, hidden) is the residual stream, updated in place (16-byte aligned); the
+// write position is kv->state[0].
+int decode_layer(fmd_dec* d, fmd_kv* kv, int l, int B, void* x, const int32_t* pad_dev,
                  const int32_t* done_dev, hipStream_t s) {
   Workspace& w = d->ws;
   DecodeLane& ln = w.dec;
   const int act = d->act;
   Layer& ly = d->layers[l];
-  void* x = w.x.p;
   AttnDecodeArgs a = attn_args(d, kv, l, B, ln.qkv.p, pad_dev, kv->state, done_dev, ln.ctx.p);
   if (qkv_in_attention(d, a, ln)) {
     a.nq = d->qkvd / 16;
@@ -245,12 +252,27 @@ int launch_logits(fmd_dec* d, const void* x, int rows, float* logits, hipStream_
   return 0;
 }
 
+// The write position and the pads of a decode call, and with ids the
+// embeddings of its tokens in ws.x, in one launch.
+int decode_setup(fmd_dec* d, fmd_kv* kv, int B, const int32_t* pad, const uint32_t* ids) {
+  DecodeSetup a{};
+  for (int b = 0; b < B; ++b) {
+    a.pad[b] = pad[b];
+    a.ids[b] = ids ? ids[b] : 0;
+  }
+  a.len = kv->len;
+  a.batch = B;
+  LAUNCH(launch_decode_setup(a, kv->state, d->ws.pad.as<int32_t>(), ids ? d->embed : nullptr,
+                             (int)(d->H * d->esz), d->ws.x.p, d->stream));
+  return 0;
+}
+
 // One decode step for B <= 16 rows: every decoder layer, then the final norm
 // fused into the lm_head projection (f32 logits + argmax keys).  Reads the
 // write position from kv->state[0].
 int decode_layers(fmd_dec* d, fmd_kv* kv, int B, const int32_t* pad_dev, const int32_t* done_dev,
                   hipStream_t s) {
-  for (int l = 0; l < d->L; ++l) CHK(decode_layer(d, kv, l, B, pad_dev, done_dev, s));
+  for (int l = 0; l < d->L; ++l) CHK(decode_layer(d, kv, l, B, d->ws.x.p, pad_dev, done_dev, s));
   return launch_logits(d, d->ws.x.p, B, d->ws.logits.as<float>(), s);
 }
 
@@ -282,7 +304,7 @@ int setup_greedy(fmd_dec* d, fmd_kv* kv, int B, int budget, const int32_t* force
   if (force)
     HIPCHK(hipMemcpyAsync(w.force.p, force, (size_t)B * 4, hipMemcpyHostToDevice, d->stream));
   CHK(kv_sync_state(kv));
-  std::memset(d->host_mirror, 0, 64);
+  std::memset(d->host_mirror, 0, kMirrorState * 4);
   return 0;
 }
 
@@ -729,7 +751,6 @@ int prefill_impl(fmd_dec* d, fmd_kv* kv, const void* emb_dev, const int32_t* pad
   CHK(launch_logits(d, w.lastx.p, B, w.logits.as<float>(), s));
   kv->len = total;
   d->logits_rows = B;
-  CHK(kv_sync_state(kv));
   return 0;
 }
 
@@ -854,10 +875,7 @@ extern "C" int fmd_dec_decode_step(fmd_dec* d, fmd_kv* kv, const uint32_t* ids, 
   HIPCHK(hipSetDevice(d->device));
   CHK(ensure_decode_ws(d, B, kv->cap));
   Workspace& w = d->ws;
-  HIPCHK(hipMemcpyAsync(w.ids.p, ids, (size_t)B * 4, hipMemcpyHostToDevice, d->stream));
-  HIPCHK(hipMemcpyAsync(w.pad.p, pad, (size_t)B * 4, hipMemcpyHostToDevice, d->stream));
-  LAUNCH(launch_embed(d->act, w.ids.as<uint32_t>(), B, d->embed, d->H, w.x.p, d->stream));
-  CHK(kv_sync_state(kv));
+  CHK(decode_setup(d, kv, B, pad, ids));
   CHK(decode_layers(d, kv, B, w.pad.as<int32_t>(), nullptr, d->stream));
   kv->len += 1;
   d->logits_rows = B;
@@ -1080,12 +1098,13 @@ extern "C" int fmd_op_layer_decode(fmd_dec* d, fmd_kv* kv, int layer, void* x, c
   HIPCHK(hipSetDevice(d->device));
   CHK(ensure_decode_ws(d, B, kv->cap));
   Workspace& w = d->ws;
+  CHK(decode_setup(d, kv, B, pad, nullptr));
+  // in place on the caller's rows where the kernels' 16-byte accesses allow it
+  const bool in_place = (uintptr_t)x % 16 == 0;
   const size_t bytes = (size_t)B * d->H * d->esz;
-  HIPCHK(hipMemcpyAsync(w.pad.p, pad, (size_t)B * 4, hipMemcpyHostToDevice, d->stream));
-  HIPCHK(hipMemcpyAsync(w.x.p, x, bytes, hipMemcpyDeviceToDevice, d->stream));
-  CHK(kv_sync_state(kv));
-  CHK(decode_layer(d, kv, layer, B, w.pad.as<int32_t>(), nullptr, d->stream));
-  HIPCHK(hipMemcpyAsync(x, w.x.p, bytes, hipMemcpyDeviceToDevice, d->stream));
+  if (!in_place) HIPCHK(hipMemcpyAsync(w.x.p, x, bytes, hipMemcpyDeviceToDevice, d->stream));
+  CHK(decode_layer(d, kv, layer, B, in_place ? x : w.x.p, w.pad.as<int32_t>(), nullptr, d->stream));
+  if (!in_place) HIPCHK(hipMemcpyAsync(x, w.x.p, bytes, hipMemcpyDeviceToDevice, d->stream));
   HIPCHK(hipStreamSynchronize(d->stream));
   return check_attn_sync(d);
 }
@@ -1231,6 +1250,7 @@ extern "C" int fmd_op_attention_decode_noalloc(fmd_dec* d, fmd_kv* kv, int layer
   AttnDecodeArgs a = attn_args(d, kv, layer, B, qkv, (const int32_t*)(base + L.pad),
                                (const int32_t*)(base + L.state), nullptr, ctx);
   a.sync = sync;
+  a.host_err = nullptr;   // this path keeps its own error words
   a.xml = a.fused ? (uint64_t*)(base + L.xml) : nullptr;
   a.xpart = a.fused ? (uint64_t*)(base + L.xpart) : nullptr;
   a.xsc = a.fused ? (uint64_t*)(base + L.xsc) : nullptr;

@@ -124,6 +124,20 @@ __global__ void embed_kernel(const uint32_t* ids, const void* table, int hidden,
   for (int i = threadIdx.x; i < hidden; i += blockDim.x) dst[i] = src[i];
 }
 
+// One work-group per row; see DecodeSetup.
+__global__ void __launch_bounds__(64) decode_setup_kernel(DecodeSetup a, int32_t* state, int32_t* pad,
+                                                          const void* table, int row_bytes, void* x) {
+  const int b = blockIdx.x, t = threadIdx.x;
+  if (b == 0) {
+    if (t < a.batch) pad[t] = a.pad[t];
+    if (t < 4) state[t] = t == 0 ? a.len : 0;
+  }
+  if (!table) return;
+  const u32x4* src = (const u32x4*)((const char*)table + (size_t)a.ids[b] * row_bytes);
+  u32x4* dst = (u32x4*)((char*)x + (size_t)b * row_bytes);
+  for (int i = t; i < row_bytes / 16; i += 64) dst[i] = src[i];
+}
+
 // Prompt assembly (MossTranscribeDiarize::splice_audio, mod.rs:128-180, then
 // the left pad of engine.rs:476-491): output row r takes src[r] >= 0 -> that
 // token's embedding, -1 -> zeros (left pad), <= -2 -> audio row -2 - src[r],
@@ -320,6 +334,14 @@ hipError_t launch_embed(int act, const uint32_t* ids, int n, const void* table, 
     case ACT_BF16: hipLaunchKernelGGL(embed_kernel<ACT_BF16>, dim3(n), dim3(256), 0, s, ids, table, hidden, out); break;
     default: return hipErrorInvalidValue;
   }
+  return hipGetLastError();
+}
+
+hipError_t launch_decode_setup(const DecodeSetup& a, int32_t* state, int32_t* pad, const void* table,
+                               int row_bytes, void* x, hipStream_t s) {
+  if (a.batch < 1 || a.batch > 16 || row_bytes % 16) return hipErrorInvalidValue;
+  hipLaunchKernelGGL(decode_setup_kernel, dim3(table ? a.batch : 1), dim3(64), 0, s, a, state, pad, table,
+                     row_bytes, x);
   return hipGetLastError();
 }
 

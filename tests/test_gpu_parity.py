@@ -229,6 +229,36 @@ def test_prefill_f16_running_reference(fmd, orc, lens, chunk):
     assert d < TOL["f16"], d
 
 
+@pytest.mark.parametrize("prec,B", [("int8", 1), ("bf16", 16)])
+def test_layer_decode_on_unaligned_rows_and_moved_lengths(fmd, prec, B):
+    """fmd_op_layer_decode runs in place on 16-byte aligned rows and through a
+    copy elsewhere: the same bits; and a length set or truncated between calls
+    is the one the next call attends to."""
+    _announce(f"layer decode alignment {prec} B={B}")
+    cfg = small_cfg(fmd, layers=1, vocab=256)
+    gpu = fmd.Qwen3(cfg, prec, max_len=512).load(fmd.synthetic_weights(cfg, seed=38))
+    dt = torch.bfloat16 if prec == "bf16" else torch.float16
+    kv = gpu.new_caches(B, 320)
+    kv.fill_random(5, 300)
+    x0 = torch.randn((B, 1024), generator=torch.Generator().manual_seed(39)).to(dt).cuda()
+    pad = [(7 * b) % 90 for b in range(B)]
+    outs = {}
+    # a call writes position `length` only: shorter lengths come later
+    for length in (300, 299, 100):
+        kv.truncate(50)
+        kv.set_len(length)
+        for off in (0, 1):
+            buf = torch.zeros(B * 1024 + 8, dtype=dt, device="cuda")
+            buf[off:off + B * 1024] = x0.reshape(-1)
+            torch.cuda.synchronize()
+            gpu.op_layer_decode(kv, 0, buf.data_ptr() + 2 * off, pad, B)
+            y = buf[off:off + B * 1024].clone()
+            assert not buf[:off].any() and not buf[off + B * 1024:].any()
+            assert torch.equal(outs.setdefault(length, y), y), (length, off)
+    assert not torch.equal(outs[300], outs[100])
+    assert kv.len() == 100
+
+
 # --------------------------------------------------------------------------
 # decode step over a synthetic padded context (configs 2 / 3 style)
 # --------------------------------------------------------------------------
