@@ -29,9 +29,9 @@ enum LinEpilogue {
 struct AffineArgs {
   const void* bias;   // (N) in the activation dtype, or NULL
   float scale;        // already rounded to the activation dtype
-  int scale_cols;     // 0: no scaling
+  int scale_cols;     // 0: no scaling; a multiple of 4
   int act;            // 0 none, 1 gelu_erf, 2 silu
-  const void* table;  // (period, N) in the activation dtype, or NULL
+  const void* table;  // (period, N) in the activation dtype, or NULL (not with a residual)
   int period, valid;
 };
 

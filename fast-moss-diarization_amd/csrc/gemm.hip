@@ -96,6 +96,20 @@ __device__ __forceinline__ void tile_of(int id, int mtiles, int cols, int a, int
   cg = (x % b) * Cb + r / gm;
 }
 
+// Four values rounded to the 16-bit activation dtype (round to nearest even).
+template <int A>
+__device__ __forceinline__ uint2 pack4(f32x4 v) {
+  if constexpr (A == ACT_BF16) {
+    typedef __bf16 b2 __attribute__((ext_vector_type(2)));
+    typedef float f2 __attribute__((ext_vector_type(2)));
+    return uint2{__builtin_bit_cast(uint32_t, __builtin_convertvector((f2){v[0], v[1]}, b2)),
+                 __builtin_bit_cast(uint32_t, __builtin_convertvector((f2){v[2], v[3]}, b2))};
+  } else {
+    return uint2{(uint32_t)st_act<A>(v[0]) | ((uint32_t)st_act<A>(v[1]) << 16),
+                 (uint32_t)st_act<A>(v[2]) | ((uint32_t)st_act<A>(v[3]) << 16)};
+  }
+}
+
 // EPI_ROPE: the work-group's 128 columns are head slot cg of q|k|v, and the
 // tile (64 or 128 rows) goes on through Attention::forward's q/k RMSNorm,
 // RoPE and KvCache::append (qwen3.rs:214-227, 139-144, 86-101) instead of
@@ -133,7 +147,9 @@ __device__ __forceinline__ RopeRows<BMT> rope_rows(const GemmArgs& p, int m0) {
 // acc: the wave's BMT/2 x 64 accumulators (2 x 2 waves, as the epilogues
 // below); stg: BMT x 128 activations of LDS, free once the caller's K loop
 // has ended.
-template <int A, int BMT, int MI>
+// CROSS: the accumulators' layout (dense tiles: see cross below); their 8-byte
+// writes (16 rows x 32 bytes) then take the swizzle R & 15.
+template <int A, int BMT, int MI, bool CROSS>
 __device__ __forceinline__ void rope_epilogue(const GemmArgs& p, const f32x4 (&acc)[MI][4],
                                               typename ActT<A>::T* stg, int m0, int cg,
                                               const RopeRows<BMT>& rr) {
@@ -159,19 +175,29 @@ __device__ __forceinline__ void rope_epilogue(const GemmArgs& p, const f32x4 (&a
     }
   }
   barrier_lds();   // every wave is done with the K loop's LDS
-  // The rows this lane writes are 4 kg + (a multiple of 4) + r, r < 4, so
-  // their rope_sw is 2 kg and column wn*64 + ni*16 + row lands at wn*64 +
-  // (ni ^ kg)*16 + row.
-  T* const wb = stg + (wm * (BMT / 2) + 4 * kg) * 128 + wn * 64 + row;
+  const int gsw = CROSS ? gi : rope_sw(gi);   // of rows gi + 16 j
+  if constexpr (CROSS) {
+    T* const wb = stg + (wm * (BMT / 2) + row) * 128 + 4 * (kg & 1);
 #pragma unroll
-  for (int mi = 0; mi < MI; ++mi)
+    for (int mi = 0; mi < MI; ++mi)
 #pragma unroll
-    for (int r = 0; r < 4; ++r)
+      for (int ni = 0; ni < 4; ++ni)
+        *(uint2*)(wb + mi * 16 * 128 + (((wn * 8 + ni * 2 + (kg >> 1)) ^ row) << 3)) =
+            pack4<A>(acc[mi][ni]);
+  } else {
+    // The rows this lane writes are 4 kg + (a multiple of 4) + r, r < 4, so
+    // their rope_sw is 2 kg and column wn*64 + ni*16 + row lands at wn*64 +
+    // (ni ^ kg)*16 + row.
+    T* const wb = stg + (wm * (BMT / 2) + 4 * kg) * 128 + wn * 64 + row;
 #pragma unroll
-      for (int ni = 0; ni < 4; ++ni) wb[(mi * 16 + r) * 128 + (ni ^ kg) * 16] = st_act<A>(acc[mi][ni][r]);
+    for (int mi = 0; mi < MI; ++mi)
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+#pragma unroll
+        for (int ni = 0; ni < 4; ++ni) wb[(mi * 16 + r) * 128 + (ni ^ kg) * 16] = st_act<A>(acc[mi][ni][r]);
+  }
   barrier_lds();
-  // rows gi + 16 j: rope_sw(gi + 16 j) = rope_sw(gi)
-  const T* const rb = stg + gi * 128 + ((dc ^ rope_sw(gi)) << 3);
+  const T* const rb = stg + gi * 128 + ((dc ^ gsw) << 3);
 #pragma unroll
   for (int j = 0; j < NJ; ++j) {
     const int gr = m0 + gi + 16 * j;
@@ -364,48 +390,6 @@ __device__ __forceinline__ void swiglu_epilogue(const GemmArgs& p, const f32x4 (
   }
 }
 
-// EPI_SWIGLU on the direct-to-LDS tiles with 16-byte stores: the same
-// products as swiglu_epilogue, staged row-major in the freed ring (BMT rows
-// x the work-group's 64 output columns; 16-byte chunk c of row R at position
-// c ^ rope_sw(R), so the four 16-lane groups' writes and the row reads are
-// bank-conflict-free), then 8 lanes per row store 8 columns each.
-template <int A, int BMT, int MI>
-__device__ __forceinline__ void swiglu_staged_epilogue(const GemmArgs& p, const f32x4 (&acc)[MI][4], int m0,
-                                                       int cg, uint16_t* stg) {
-  typedef typename ActT<A>::T T;
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-  const int wm = w >> 1, wn = w & 1, row = lane & 15, kg = lane >> 4;
-  barrier_lds();   // every wave's last fragment reads are done
-#pragma unroll
-  for (int mi = 0; mi < MI; ++mi) {
-    float o[4][2];
-#pragma unroll
-    for (int r = 0; r < 4; ++r)
-#pragma unroll
-      for (int ni = 0; ni < 2; ++ni) {
-        const float gg = rd<A>(acc[mi][ni][r]), u = rd<A>(acc[mi][ni + 2][r]);
-        o[r][ni] = rd<A>(gg / (1.0f + __expf(-gg))) * u;
-      }
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int R = wm * (BMT / 2) + mi * 16 + 4 * kg + r;
-#pragma unroll
-      for (int ni = 0; ni < 2; ++ni) {
-        const int C = (wn * 2 + ni) * 16 + row;
-        stg[R * 64 + ((((C >> 3) ^ rope_sw(R)) << 3) | (C & 7))] = st_act<A>(o[r][ni]);
-      }
-    }
-  }
-  barrier_lds();
-  const int ch = threadIdx.x & 7, r0 = threadIdx.x >> 3;    // chunk, first row
-  const int gc = cg * 64 + ch * 8;                           // its first output column
-  if (gc >= p.W.out / 2) return;                             // (no barrier follows)
-  const int rows = min(BMT, p.M - m0);
-  T* const y = (T*)p.y + (size_t)m0 * p.ldy + gc;
-  for (int R = r0; R < rows; R += 32)
-    *(u32x4*)(y + (size_t)R * p.ldy) = *(const u32x4*)&stg[R * 64 + ((ch ^ rope_sw(R)) << 3)];
-}
-
 // Q8_0 weights (f16 activations) past the small grids: 64 x 128 tiles, K step
 // 64, X staged global -> registers -> LDS, weight fragments and scales read
 // straight from global memory one K step ahead.  The tiles scale each block's
@@ -548,7 +532,7 @@ gemm_q8_kernel(GemmArgs p) {
   }
 
   if constexpr (EPI == EPI_ROPE) {
-    rope_epilogue<A, BMT, MI>(p, acc, sA, m0, cg, rrows);
+    rope_epilogue<A, BMT, MI, false>(p, acc, sA, m0, cg, rrows);
     return;
   }
   if constexpr (EPI == EPI_SWIGLU) {
@@ -588,12 +572,6 @@ gemm_q8_kernel(GemmArgs p) {
 // work-groups per CU at (128, 4) and (256, 3), three at (64, 4).
 constexpr int BK2 = 32;
 
-// EPI_SWIGLU with 16-byte stores on the direct-to-LDS tiles (the host picks
-// it when the output allows them).
-constexpr int EPI_SWIGLU_STAGED = 102;
-
-
-
 __device__ __forceinline__ int swz(int r) { return ((r >> 1) ^ (r >> 3)) & 3; }
 
 // Two values already rounded to the 16-bit activation dtype, packed (lo in
@@ -605,6 +583,134 @@ __device__ __forceinline__ uint32_t pack2_rounded(float lo, float hi) {
     return __builtin_amdgcn_perm(__builtin_bit_cast(uint32_t, hi), __builtin_bit_cast(uint32_t, lo), 0x07060302u);
   else
     return (uint32_t)st_act<A>(lo) | ((uint32_t)st_act<A>(hi) << 16);
+}
+
+// Dense tiles run their MFMAs with the weights as the A operand (both operands'
+// fragments have the same layout), Y^T = W X^T per 16 x 16 piece: a lane then
+// holds four consecutive output columns 4 kg .. 4 kg + 3 of tile[ni] for X row
+// 16 mi + lane % 16, so residuals, tables and outputs move 8 bytes at a time
+// straight from the registers, and what is staged through LDS is written 8
+// bytes at a time.  Against 2-byte accesses in the other layout (the same
+// bits): encoder layer at 16 windows 936 -> 927 us, 5 x 1137 306.5 -> 304.4 us.
+
+// Four consecutive 16-bit values at q (VEC: 8-byte aligned).
+template <bool VEC>
+__device__ __forceinline__ uint2 load4(const uint16_t* q) {
+  if constexpr (VEC) return *(const uint2*)q;
+  else return uint2{q[0] | ((uint32_t)q[1] << 16), q[2] | ((uint32_t)q[3] << 16)};
+}
+template <bool VEC>
+__device__ __forceinline__ void store4(uint16_t* q, uint2 v) {
+  if constexpr (VEC) {
+    *(uint2*)q = v;
+  } else {
+    q[0] = (uint16_t)v.x;
+    q[1] = (uint16_t)(v.x >> 16);
+    q[2] = (uint16_t)v.y;
+    q[3] = (uint16_t)(v.y >> 16);
+  }
+}
+__device__ __forceinline__ uint16_t elem4(uint2 v, int r) {
+  return (uint16_t)((r < 2 ? v.x : v.y) >> (16 * (r & 1)));
+}
+
+// The residual, or the table value, of every output a lane stores (a product
+// has at most one of the two; with neither, unused values of y); rows past M
+// and tiles past the end read clamped addresses (they are not stored).  mb: the
+// wave's first row.
+template <bool VEC, int MI, int NI>
+__device__ __forceinline__ void cross_resid(const GemmArgs& p, int mb, const int (&tile)[NI], const bool (&tv)[NI],
+                                            uint2 (&rr)[MI][NI]) {
+  const int lane = threadIdx.x & 63, row = lane & 15, kg = lane >> 4;
+  const bool tab = !p.resid && p.aff.table;
+  const uint16_t* rp = (const uint16_t*)(p.resid ? p.resid : tab ? p.aff.table : p.y) + 4 * kg;
+  const int ld = tab ? p.W.out : p.ldy;
+#pragma unroll
+  for (int mi = 0; mi < MI; ++mi) {
+    int r = min(mb + mi * 16 + row, p.M - 1);
+    if (tab) r = min(r % p.aff.period, p.aff.valid - 1);
+#pragma unroll
+    for (int ni = 0; ni < NI; ++ni) rr[mi][ni] = load4<VEC>(rp + (size_t)r * ld + (tv[ni] ? tile[ni] : 0) * 16);
+  }
+}
+
+// Epilogue of a wave's MI x NI pieces (EPI_STORE, RESID, SWIGLU, AFFINE).
+// SWIGLU: tiles [0, NI / 2) hold gate columns, the others the matching up
+// columns.  rr: cross_resid's values (EPI_RESID, and EPI_AFFINE with a
+// residual or a table; every load comes before the first store, since a vector-memory wait
+// also counts the stores issued before it).
+template <int A, int EPI, bool VEC, int MI, int NI>
+__device__ __forceinline__ void cross_epilogue(const GemmArgs& p, const f32x4 (&acc)[MI][NI], int mb,
+                                               const int (&tile)[NI], const bool (&tv)[NI],
+                                               const uint2 (&rr)[MI][NI]) {
+  const int lane = threadIdx.x & 63, row = lane & 15, kg = lane >> 4;
+  uint16_t* const y = (uint16_t*)p.y + 4 * kg;
+  if constexpr (EPI == EPI_SWIGLU) {
+    constexpr int G = NI / 2;
+#pragma unroll
+    for (int mi = 0; mi < MI; ++mi) {
+      f32x4 o[G];
+#pragma unroll
+      for (int ni = 0; ni < G; ++ni)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const float gg = rd<A>(acc[mi][ni][r]), u = rd<A>(acc[mi][ni + G][r]);
+          o[ni][r] = rd<A>(gg / (1.0f + __expf(-gg))) * u;
+        }
+      const int gr = mb + mi * 16 + row;
+#pragma unroll
+      for (int ni = 0; ni < G; ++ni)
+        if (gr < p.M && tv[ni]) store4<VEC>(y + (size_t)gr * p.ldy + tile[ni] * 16, pack4<A>(o[ni]));
+    }
+  } else if constexpr (EPI == EPI_AFFINE) {
+    const AffineArgs& f = p.aff;
+    constexpr int N = NI * 4;
+    float bs[N], sc[NI];
+#pragma unroll
+    for (int ni = 0; ni < NI; ++ni) {
+      const int col = (tv[ni] ? tile[ni] : 0) * 16 + 4 * kg;
+      const uint2 b = f.bias ? load4<VEC>((const uint16_t*)f.bias + col) : uint2{0, 0};
+#pragma unroll
+      for (int r = 0; r < 4; ++r) bs[ni * 4 + r] = ld_act<A>(elem4(b, r));
+      sc[ni] = col < f.scale_cols ? f.scale : 1.0f;   // scale_cols is a multiple of 4
+    }
+#pragma unroll
+    for (int mi = 0; mi < MI; ++mi) {
+      float v[N], sv[N];
+      uint16_t xv[N];
+#pragma unroll
+      for (int e = 0; e < N; ++e) {
+        v[e] = acc[mi][e >> 2][e & 3];
+        sv[e] = sc[e >> 2];
+        xv[e] = elem4(rr[mi][e >> 2], e & 3);
+      }
+      affine_block<A, N, false>(p, v, sv, bs, xv, xv);
+      const int gr = mb + mi * 16 + row;
+      if (gr >= p.M || !affine_row(p, gr)) continue;
+      uint16_t* const yr = y + (size_t)gr * p.ldy;
+#pragma unroll
+      for (int ni = 0; ni < NI; ++ni)
+        if (tv[ni])
+          store4<VEC>(yr + tile[ni] * 16, uint2{pack2_rounded<A>(v[4 * ni], v[4 * ni + 1]),
+                                                pack2_rounded<A>(v[4 * ni + 2], v[4 * ni + 3])});
+    }
+  } else {
+#pragma unroll
+    for (int mi = 0; mi < MI; ++mi) {
+      const int gr = mb + mi * 16 + row;
+      if (gr >= p.M) continue;
+#pragma unroll
+      for (int ni = 0; ni < NI; ++ni) {
+        if (!tv[ni]) continue;
+        f32x4 v = acc[mi][ni];
+        if constexpr (EPI == EPI_RESID) {
+#pragma unroll
+          for (int r = 0; r < 4; ++r) v[r] = ld_act<A>(elem4(rr[mi][ni], r)) + rd<A>(v[r]);
+        }
+        store4<VEC>(y + (size_t)gr * p.ldy + tile[ni] * 16, pack4<A>(v));
+      }
+    }
+  }
 }
 
 // EPI_AFFINE on the direct-to-LDS BMT x 128 tiles, through LDS: the
@@ -628,7 +734,7 @@ __device__ __forceinline__ void staged_affine_epilogue(const GemmArgs& p, const 
   const bool col_ok = gc < p.W.out;
   const int rows = min(BMT, p.M - m0);
   // The bias and the residual or table values (a product has at most one
-  // of the two: staged_ok) of the lane's rows r0, r0 + 16, ... are loaded
+  // of the two) of the lane's rows r0, r0 + 16, ... are loaded
   // first, so the loads run under the staging below and none follows a
   // store: a vector-memory wait also counts the stores issued before it, so
   // a load placed after a store would hold the lane until that store
@@ -660,17 +766,15 @@ __device__ __forceinline__ void staged_affine_epilogue(const GemmArgs& p, const 
     xv4[i] = *(const u32x4*)(xb + (size_t)xr * xs);
   }
   barrier_lds();   // every wave's last fragment reads are done
+  {
+    uint16_t* const wb = stg + (wm * (BMT / 2) + row) * 128 + 4 * (kg & 1);
 #pragma unroll
-  for (int mi = 0; mi < MI; ++mi)
+    for (int mi = 0; mi < MI; ++mi)
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int R = wm * (BMT / 2) + mi * 16 + 4 * kg + r;
-#pragma unroll
-      for (int ni = 0; ni < 4; ++ni) {
-        const int C = wn * 64 + ni * 16 + row;
-        stg[R * 128 + ((((C >> 3) ^ rope_sw(R)) << 3) | (C & 7))] = st_act<A>(acc[mi][ni][r]);
-      }
-    }
+      for (int ni = 0; ni < 4; ++ni)
+        *(uint2*)(wb + mi * 16 * 128 + (((wn * 8 + ni * 2 + (kg >> 1)) ^ row) << 3)) =
+            pack4<A>(acc[mi][ni]);
+  }
   barrier_lds();
   if (!col_ok) return;                                       // (no barrier follows)
   T* const y = (T*)p.y + (size_t)m0 * p.ldy + gc;
@@ -687,7 +791,7 @@ __device__ __forceinline__ void staged_affine_epilogue(const GemmArgs& p, const 
 #pragma unroll
     for (int q = 0; q < 2; ++q) {
       const int R = min(r0 + 16 * (i + q), rows - 1);
-      unpack8<A>(*(const u32x4*)&stg[R * 128 + ((ch ^ rope_sw(R)) << 3)], &v[8 * q]);
+      unpack8<A>(*(const u32x4*)&stg[R * 128 + ((ch ^ (R & 15)) << 3)], &v[8 * q]);
 #pragma unroll
       for (int e = 0; e < 8; ++e) {
         xv[8 * q + e] = (T)(xv4[i + q][e / 2] >> (16 * (e & 1)));
@@ -718,15 +822,14 @@ gemm_dma_kernel(GemmArgs p) {
   constexpr int PER = NX + 2;            // copies per thread per stage
   constexpr int SA = BMT * BK2;          // X elements per stage
   constexpr int SB = 8 * 512;            // weight elements per stage (8 KB)
-  static_assert(NS * (SA + SB) >= BMT * 128, "the staged epilogue reuses the ring");
+  static_assert(NS * (SA + SB) >= BMT * 128, "the staged epilogues reuse the ring");
   __shared__ __attribute__((aligned(1024))) uint16_t smem[NS * (SA + SB)];
   uint16_t* const sA = smem;
   uint16_t* const sB = smem + NS * SA;
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
   const int wm = w >> 1, wn = w & 1;
   const int K = p.W.in, ntiles = p.W.out / 16;
-  constexpr int WEPI = EPI == EPI_SWIGLU_STAGED ? EPI_SWIGLU : EPI;   // the tiles' layout
-  const int cols = WEPI == EPI_SWIGLU ? (ntiles / 2 + 3) / 4 : (ntiles + 7) / 8;
+  const int cols = EPI == EPI_SWIGLU ? (ntiles / 2 + 3) / 4 : (ntiles + 7) / 8;
   int mt, cg;
   tile_of(blockIdx.x, (p.M + BMT - 1) / BMT, cols, p.map, mt, cg);
   if (mt * BMT >= p.M) return;
@@ -738,12 +841,13 @@ gemm_dma_kernel(GemmArgs p) {
   bool tv[4];
 #pragma unroll
   for (int ni = 0; ni < 4; ++ni) {
-    tile[ni] = wave_tile<WEPI>(cg, ntiles, wn, ni);
-    tv[ni] = (WEPI == EPI_SWIGLU) ? (cg * 4 + wn * 2 + (ni & 1)) < ntiles / 2 : tile[ni] < ntiles;
+    tile[ni] = wave_tile<EPI>(cg, ntiles, wn, ni);
+    tv[ni] = (EPI == EPI_SWIGLU) ? (cg * 4 + wn * 2 + (ni & 1)) < ntiles / 2 : tile[ni] < ntiles;
   }
+  const int mb = m0 + wm * (BMT / 2);
+  [[maybe_unused]] uint2 rres[MI][4];   // in flight behind the K loop
   static_assert(EPI != EPI_RESID || BMT <= 128, "residual prefetch: 64- and 128-row tiles");
-  [[maybe_unused]] ResidRows<A, EPI == EPI_RESID ? MI : 1> rres;
-  if constexpr (EPI == EPI_RESID) rres = load_resid<A, BMT, MI>(p, m0, tile, tv);
+  if constexpr (EPI == EPI_RESID) cross_resid<true, MI, 4>(p, mb, tile, tv, rres);
   // This thread's copies per stage: X slots j * 64 + lane of instructions
   // j = NX w .. NX w + NX - 1 (rows 16 j + lane / 4; rows past M read row
   // M - 1), weight tiles t = 2w, 2w + 1 (past the end: the last tile).
@@ -759,8 +863,8 @@ gemm_dma_kernel(GemmArgs p) {
 #pragma unroll
   for (int i = 0; i < 2; ++i) {
     const int t = 2 * w + i;
-    int tl = wave_tile<WEPI>(cg, ntiles, t >> 2, t & 3);
-    const bool ok = (WEPI == EPI_SWIGLU) ? (cg * 4 + (t >> 2) * 2 + (t & 1)) < ntiles / 2 : tl < ntiles;
+    int tl = wave_tile<EPI>(cg, ntiles, t >> 2, t & 3);
+    const bool ok = (EPI == EPI_SWIGLU) ? (cg * 4 + (t >> 2) * 2 + (t & 1)) < ntiles / 2 : tl < ntiles;
     tl = ok ? tl : ntiles - 1;
     woff[i] = ((uint32_t)tl * (K / 32) * 64 + lane) * 16u;
   }
@@ -807,42 +911,16 @@ gemm_dma_kernel(GemmArgs p) {
       const int r = wm * (BMT / 2) + mi * 16 + row;
       const u32x4 fa = *(const u32x4*)&a[(r * 4 + (kg ^ swz(r))) * 8];
 #pragma unroll
-      for (int ni = 0; ni < 4; ++ni) acc[mi][ni] = mfma16<A>(fa, fb[ni], acc[mi][ni]);
+      for (int ni = 0; ni < 4; ++ni) acc[mi][ni] = mfma16<A>(fb[ni], fa, acc[mi][ni]);
     }
   }
 
   if constexpr (EPI == EPI_ROPE) {
-    rope_epilogue<A, BMT, MI>(p, acc, sA, m0, cg, rrows);
-    return;
-  }
-  if constexpr (EPI == EPI_AFFINE) {
+    rope_epilogue<A, BMT, MI, true>(p, acc, smem, m0, cg, rrows);
+  } else if constexpr (EPI == EPI_AFFINE) {
     staged_affine_epilogue<A, BMT, MI>(p, acc, m0, cg, smem);
-    return;
-  }
-  if constexpr (EPI == EPI_SWIGLU_STAGED) {
-    swiglu_staged_epilogue<A, BMT, MI>(p, acc, m0, cg, smem);
-    return;
-  }
-  if constexpr (EPI == EPI_SWIGLU) {
-    swiglu_epilogue<A, BMT, MI>(p, acc, m0, tile, tv);
-    return;
-  }
-#pragma unroll
-  for (int mi = 0; mi < MI; ++mi) {
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int gr = m0 + wm * (BMT / 2) + mi * 16 + 4 * kg + r;
-      if (gr >= p.M) continue;
-#pragma unroll
-      for (int ni = 0; ni < 4; ++ni) {
-        if (!tv[ni]) continue;
-        const size_t o = (size_t)gr * p.ldy + tile[ni] * 16 + row;
-        if constexpr (EPI == EPI_RESID)
-          ((T*)p.y)[o] = st_act<A>(ld_act<A>(rres.v[mi][r][ni]) + rd<A>(acc[mi][ni][r]));
-        else
-          ((T*)p.y)[o] = st_act<A>(acc[mi][ni][r]);
-      }
-    }
+  } else {
+    cross_epilogue<A, EPI, true, MI, 4>(p, acc, mb, tile, tv, rres);
   }
 }
 
@@ -891,7 +969,7 @@ __device__ __forceinline__ int small_tile(int cg, int ntiles, int lt, bool& ok) 
   }
 }
 
-template <int A, int WK, int EPI, int BM, int BN, int KS, int NS>
+template <int A, int WK, int EPI, int BM, int BN, int KS, int NS, bool VEC>
 __global__ void __launch_bounds__(256) gemm_small_kernel(GemmArgs p) {
   typedef typename ActT<A>::T T;
   constexpr bool Q8 = WK == WK_Q8;
@@ -928,18 +1006,19 @@ __global__ void __launch_bounds__(256) gemm_small_kernel(GemmArgs p) {
 
   // The residuals of the elements this lane stores, loaded before the K loop
   // (rows past M and tiles past the end read clamped addresses).
-  constexpr bool RES = EPI == EPI_RESID || EPI == EPI_AFFINE;
-  [[maybe_unused]] T rres[RES ? MI * 4 * NI : 1];
-  if constexpr (RES) {
-    const T* rp = (const T*)(p.resid ? p.resid : p.y);
+  const int mb = m0 + wm * (BM / 2);
+  [[maybe_unused]] uint2 rres[Q8 ? 1 : MI][NI];          // dense
+  [[maybe_unused]] T qres[Q8 ? MI : 1][4][Q8 ? NI : 1];  // Q8_0: rows 4 kg + r, column `row`
+  if constexpr (!Q8 && (EPI == EPI_RESID || EPI == EPI_AFFINE)) cross_resid<VEC, MI, NI>(p, mb, tile, tv, rres);
+  if constexpr (Q8 && EPI == EPI_RESID) {
 #pragma unroll
     for (int mi = 0; mi < MI; ++mi)
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
-        const int gr = min(m0 + wm * (BM / 2) + mi * 16 + 4 * kg + r, p.M - 1);
+        const int gr = min(mb + mi * 16 + 4 * kg + r, p.M - 1);
 #pragma unroll
         for (int ni = 0; ni < NI; ++ni)
-          rres[(mi * 4 + r) * NI + ni] = rp[(size_t)gr * p.ldy + (tv[ni] ? tile[ni] : 0) * 16 + row];
+          qres[mi][r][ni] = ((const T*)p.resid)[(size_t)gr * p.ldy + (tv[ni] ? tile[ni] : 0) * 16 + row];
       }
   }
 
@@ -1046,7 +1125,7 @@ __global__ void __launch_bounds__(256) gemm_small_kernel(GemmArgs p) {
           const int r = wm * (BM / 2) + mi * 16 + row;
           const u32x4 fa = *(const u32x4*)&a[r * KS + (((4 * ks + kg) ^ swx<KS>(r)) << 3)];
 #pragma unroll
-          for (int ni = 0; ni < NI; ++ni) acc[mi][ni] = mfma16<A>(fa, fb[ni], acc[mi][ni]);
+          for (int ni = 0; ni < NI; ++ni) acc[mi][ni] = mfma16<A>(fb[ni], fa, acc[mi][ni]);
         }
       }
     }
@@ -1054,75 +1133,30 @@ __global__ void __launch_bounds__(256) gemm_small_kernel(GemmArgs p) {
   }
 
   if constexpr (EPI == EPI_ROPE) {
-    rope_epilogue<A, BM, MI>(p, acc, (T*)smem, m0, cg, rrows);
-    return;
-  }
-  if constexpr (EPI == EPI_SWIGLU) {
-    constexpr int G = NI / 2;
+    rope_epilogue<A, BM, MI, !Q8>(p, acc, (T*)smem, m0, cg, rrows);
+  } else if constexpr (!Q8) {
+    cross_epilogue<A, EPI, VEC, MI, NI>(p, acc, mb, tile, tv, rres);
+  } else {
+    // Q8_0 (each column's block scale sits in the lane of that column): a lane
+    // holds rows 4 kg + r of each fragment, column `row`
+    constexpr int NO = EPI == EPI_SWIGLU ? NI / 2 : NI;
 #pragma unroll
     for (int mi = 0; mi < MI; ++mi)
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
-        const int gr = m0 + wm * (BM / 2) + mi * 16 + 4 * kg + r;
+        const int gr = mb + mi * 16 + 4 * kg + r;
 #pragma unroll
-        for (int ni = 0; ni < G; ++ni) {
-          const float gg = rd<A>(acc[mi][ni][r]), u = rd<A>(acc[mi][ni + G][r]);
-          const float o = rd<A>(gg / (1.0f + __expf(-gg))) * u;
-          if (gr < p.M && tv[ni]) ((T*)p.y)[(size_t)gr * p.ldy + tile[ni] * 16 + row] = st_act<A>(o);
+        for (int ni = 0; ni < NO; ++ni) {
+          float v = acc[mi][ni][r];
+          if constexpr (EPI == EPI_SWIGLU) {
+            const float gg = rd<A>(v), u = rd<A>(acc[mi][ni + NO][r]);
+            v = rd<A>(gg / (1.0f + __expf(-gg))) * u;
+          }
+          if constexpr (EPI == EPI_RESID) v = ld_act<A>(qres[mi][r][ni]) + rd<A>(v);
+          if (gr < p.M && tv[ni]) ((T*)p.y)[(size_t)gr * p.ldy + tile[ni] * 16 + row] = st_act<A>(v);
         }
       }
-    return;
   }
-  if constexpr (EPI == EPI_AFFINE) {
-    constexpr int N = MI * 4 * NI;
-    float v[N], sc[N], bs[N];
-    T tb[N];
-#pragma unroll
-    for (int ni = 0; ni < NI; ++ni) {
-      const int col = (tv[ni] ? tile[ni] : 0) * 16 + row;
-      const float b = p.aff.bias ? ld_act<A>(((const T*)p.aff.bias)[col]) : 0.f;
-      const float s1 = col < p.aff.scale_cols ? p.aff.scale : 1.f;
-#pragma unroll
-      for (int mi = 0; mi < MI; ++mi)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          const int e = (mi * 4 + r) * NI + ni;
-          const int gr = min(m0 + wm * (BM / 2) + mi * 16 + 4 * kg + r, p.M - 1);
-          v[e] = acc[mi][ni][r];
-          bs[e] = b;
-          sc[e] = s1;
-          tb[e] = p.aff.table ? ((const T*)p.aff.table)[(size_t)min(gr % p.aff.period, p.aff.valid - 1) * p.W.out + col] : (T)0;
-        }
-    }
-    affine_block<A, N, false>(p, v, sc, bs, rres, tb);
-#pragma unroll
-    for (int mi = 0; mi < MI; ++mi)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int gr = m0 + wm * (BM / 2) + mi * 16 + 4 * kg + r;
-        if (gr >= p.M || !affine_row(p, gr)) continue;
-#pragma unroll
-        for (int ni = 0; ni < NI; ++ni)
-          if (tv[ni]) ((T*)p.y)[(size_t)gr * p.ldy + tile[ni] * 16 + row] = st_act<A>(v[(mi * 4 + r) * NI + ni]);
-      }
-    return;
-  }
-#pragma unroll
-  for (int mi = 0; mi < MI; ++mi)
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int gr = m0 + wm * (BM / 2) + mi * 16 + 4 * kg + r;
-      if (gr >= p.M) continue;
-#pragma unroll
-      for (int ni = 0; ni < NI; ++ni) {
-        if (!tv[ni]) continue;
-        const size_t o = (size_t)gr * p.ldy + tile[ni] * 16 + row;
-        if constexpr (EPI == EPI_RESID)
-          ((T*)p.y)[o] = st_act<A>(ld_act<A>(rres[(mi * 4 + r) * NI + ni]) + rd<A>(acc[mi][ni][r]));
-        else
-          ((T*)p.y)[o] = st_act<A>(acc[mi][ni][r]);
-      }
-    }
 }
 
 // f32 activations / weights on v_mfma_f32_16x16x4f32; same tiling, K chunks of 16.
@@ -1231,12 +1265,11 @@ GemmTile gemm_tile(int M, int col_groups) {
   return TILE64;
 }
 
-// 16-byte output, bias, residual and table accesses for the staged
-// epilogues, which also hold a residual or a table, not both.
-bool staged_ok(const GemmArgs& a) {
+// Whether the dense tiles may move 16 bytes of output, bias, residual and table
+// rows at a time.
+bool vec_ok(const GemmArgs& a) {
   auto al = [](const void* q) { return ((uintptr_t)q & 15) == 0; };
-  return !(a.resid && a.aff.table) && a.ldy % 8 == 0 && al(a.y) && (!a.aff.bias || al(a.aff.bias)) &&
-         (!a.aff.table || al(a.aff.table)) && (!a.resid || al(a.resid)) && a.W.out % 8 == 0;
+  return a.ldy % 8 == 0 && al(a.y) && al(a.aff.bias) && al(a.aff.table) && al(a.resid);
 }
 
 template <int A, int BMT, int NS>
@@ -1247,18 +1280,12 @@ hipError_t launch_dma(int epi, dim3 grid, const GemmArgs& a, hipStream_t s) {
       if constexpr (BMT > 128) return hipErrorInvalidValue;
       else hipLaunchKernelGGL((gemm_dma_kernel<A, EPI_RESID, BMT, NS>), grid, dim3(256), 0, s, a);
       break;
-    case EPI_SWIGLU:
-      if (staged_ok(a)) hipLaunchKernelGGL((gemm_dma_kernel<A, EPI_SWIGLU_STAGED, BMT, NS>), grid, dim3(256), 0, s, a);
-      else hipLaunchKernelGGL((gemm_dma_kernel<A, EPI_SWIGLU, BMT, NS>), grid, dim3(256), 0, s, a);
-      break;
+    case EPI_SWIGLU: hipLaunchKernelGGL((gemm_dma_kernel<A, EPI_SWIGLU, BMT, NS>), grid, dim3(256), 0, s, a); break;
     case EPI_ROPE:
       if constexpr (BMT > 128) return hipErrorInvalidValue;
       else hipLaunchKernelGGL((gemm_dma_kernel<A, EPI_ROPE, BMT, NS>), grid, dim3(256), 0, s, a);
       break;
-    case EPI_AFFINE:
-      if (!staged_ok(a)) return hipErrorInvalidValue;  // try_small takes these
-      hipLaunchKernelGGL((gemm_dma_kernel<A, EPI_AFFINE, BMT, NS>), grid, dim3(256), 0, s, a);
-      break;
+    case EPI_AFFINE: hipLaunchKernelGGL((gemm_dma_kernel<A, EPI_AFFINE, BMT, NS>), grid, dim3(256), 0, s, a); break;
     default: return hipErrorInvalidValue;
   }
   return hipGetLastError();
@@ -1292,7 +1319,7 @@ int xcd_rows(const GemmArgs& p, int cols, int bm) {
   return best;
 }
 
-template <int A, int WK, int BM, int BN, int KS, int NS>
+template <int A, int WK, int BM, int BN, int KS, int NS, bool VEC = true>
 hipError_t launch_small(int epi, const GemmArgs& a, hipStream_t s) {
   const int ntiles = a.W.out / 16;
   const int cw = epi == EPI_SWIGLU ? BN / 32 : BN / 16;
@@ -1301,22 +1328,22 @@ hipError_t launch_small(int epi, const GemmArgs& a, hipStream_t s) {
   g.map = xcd_rows(a, cols, BM);
   const int mtiles = (a.M + BM - 1) / BM, Ma = (mtiles + g.map - 1) / g.map;
   const dim3 grid(8 * Ma * (cols / (8 / g.map)));
-#define SMALL(E) hipLaunchKernelGGL((gemm_small_kernel<A, WK, E, BM, BN, KS, NS>), grid, dim3(256), 0, s, g)
+#define SMALL(E) hipLaunchKernelGGL((gemm_small_kernel<A, WK, E, BM, BN, KS, NS, VEC>), grid, dim3(256), 0, s, g)
   switch (epi) {
+    case EPI_STORE:
+      if constexpr (BN < 128) { SMALL(EPI_STORE); break; }
+      return hipErrorInvalidValue;
     case EPI_ROPE:
       if constexpr (BN == 128) { SMALL(EPI_ROPE); break; }
       return hipErrorInvalidValue;
     case EPI_SWIGLU:
-      if constexpr (BN == 64) { SMALL(EPI_SWIGLU); break; }
+      if constexpr (BN == 64 && VEC) { SMALL(EPI_SWIGLU); break; }
       return hipErrorInvalidValue;
     case EPI_AFFINE:   // the audio path is dense
-      if constexpr (BN < 128 && WK != WK_Q8) { SMALL(EPI_AFFINE); break; }
-      return hipErrorInvalidValue;
-    case EPI_STORE:
-      if constexpr (BN < 128) { SMALL(EPI_STORE); break; }
+      if constexpr (BN < 128 && WK != WK_Q8 && VEC) { SMALL(EPI_AFFINE); break; }
       return hipErrorInvalidValue;
     case EPI_RESID:
-      if constexpr (BN < 128) { SMALL(EPI_RESID); break; }
+      if constexpr (BN < 128 && VEC) { SMALL(EPI_RESID); break; }
       return hipErrorInvalidValue;
     default: return hipErrorInvalidValue;
   }
@@ -1355,14 +1382,15 @@ bool try_small(int epi, const GemmArgs& a, hipStream_t s, hipError_t* e) {
     else if (!n64 && fits(32, 128, 128, 256)) *e = launch_small<A, WK, 32, 128, 128, 3>(epi, a, s);
     else return false;
   } else {
-    // the direct-to-LDS tiles' affine epilogue moves 16 bytes at a time; an
-    // output, residual, bias or table that does not allow it stays here
-    const bool stay = epi == EPI_AFFINE && !staged_ok(a);
-    if (n32 && fits(32, 32, 128, 256)) *e = launch_small<A, WK, 32, 32, 128, 4>(epi, a, s);
+    // a caller's unaligned output (EPI_STORE only: every other product works on
+    // the library's buffers) is stored element by element, by one tile kind
+    if (epi == EPI_STORE && !vec_ok(a)) *e = launch_small<A, WK, 128, 64, 64, 3, false>(epi, a, s);
+    else if (epi != EPI_ROPE && !vec_ok(a)) *e = hipErrorInvalidValue;
+    else if (n32 && fits(32, 32, 128, 256)) *e = launch_small<A, WK, 32, 32, 128, 4>(epi, a, s);
     else if (n64 && fits(32, 64, 128, 256)) *e = launch_small<A, WK, 32, 64, 128, 3>(epi, a, s);
     else if (n64 && fits(64, 64, 128, 256)) *e = launch_small<A, WK, 64, 64, 128, 3>(epi, a, s);
     else if (n64 && fits(64, 64, 64, 512)) *e = launch_small<A, WK, 64, 64, 64, 4>(epi, a, s);
-    else if (n64 && (stay || fits(128, 64, 64, 512))) *e = launch_small<A, WK, 128, 64, 64, 3>(epi, a, s);
+    else if (n64 && fits(128, 64, 64, 512)) *e = launch_small<A, WK, 128, 64, 64, 3>(epi, a, s);
     else if (!n64 && fits(32, 128, 64, 256)) *e = launch_small<A, WK, 32, 128, 64, 4>(epi, a, s);
     else if (!n64 && fits(64, 128, 64, 512)) *e = launch_small<A, WK, 64, 128, 64, 3>(epi, a, s);
     else return false;
@@ -1422,7 +1450,8 @@ hipError_t launch_gemm(int act, int epi, const GemmArgs& a, hipStream_t s) {
     return hipErrorInvalidValue;
   if (epi == EPI_AFFINE && ((a.aff.table && (a.aff.period <= 0 || a.aff.valid < 1)) ||
                             (a.aff.period > 0 && (a.aff.valid < 0 || a.aff.valid > a.aff.period)) ||
-                            a.aff.act < 0 || a.aff.act > 2 || a.aff.scale_cols < 0))
+                            a.aff.act < 0 || a.aff.act > 2 || a.aff.scale_cols < 0 ||
+                            a.aff.scale_cols % 4 || (a.resid && a.aff.table)))
     return hipErrorInvalidValue;
   if (a.W.kind == WK_Q8) {
     if (act != ACT_F16) return hipErrorInvalidValue;

@@ -184,6 +184,13 @@ def test_linear_tile_kinds_give_the_same_bits(fmd, prec):
             gpu.op_linear(0, proj, x.data_ptr(), m, y.data_ptr())
             torch.cuda.synchronize()
             assert torch.equal(y, full[:m]), (proj, m)
+        for m in (100, 4300):   # an output that allows 2-byte stores only
+            buf = torch.zeros(m * n + 8, dtype=dt, device="cuda")
+            torch.cuda.synchronize()
+            gpu.op_linear(0, proj, x.data_ptr(), m, buf.data_ptr() + 2)
+            torch.cuda.synchronize()
+            assert torch.equal(buf[1:1 + m * n].reshape(m, n), full[:m]), (proj, m)
+            assert not buf[:1].any() and not buf[1 + m * n:].any()
 
 
 @pytest.mark.parametrize("prec,n", [("int8", 20), ("int8", 225), ("int8", 450), ("f16", 65),
