@@ -161,15 +161,19 @@ int ensure_ws(fmd_enc* e, int windows, int t, int frames) {
   return 0;
 }
 
-// The layers [first, first + n) and (final_norm) the final LayerNorm over the
-// rows of e->x (windows of t positions, t + 1 rows apart); the normalised
-// rows go to `out` (windows * t rows of d, contiguous, device).
-int run_layers(fmd_enc* e, int windows, int t, int first, int n, bool final_norm, void* out) {
+// The layers [first, first + n) and (final_norm) the final LayerNorm over
+// windows of t positions, P rows apart.  The first layer reads `in` (windows * P
+// rows of d, device, left as it is; the others work in e->x, which may be `in`)
+// and the last result goes to `out` (windows * P rows; e->x or another buffer,
+// also `in`: it is written last).  in and out are 16-byte aligned.
+int run_layers(fmd_enc* e, int windows, int t, int P, int first, int n, bool final_norm, const void* in,
+               void* out) {
   hipStream_t s = e->stream;
-  const int P = t + 1, rows = windows * P, d = e->d, act = e->act;
+  const int rows = windows * P, d = e->d, act = e->act;
+  const void* x = in;   // the residual stream
   for (int l = first; l < first + n; ++l) {
     const EncLayer& L = e->layers[l];
-    LAUNCH(launch_layernorm(act, e->x.p, d, L.ln1_w, L.ln1_b, rows, d, kLnEps, e->xn.p, d, s));
+    LAUNCH(launch_layernorm(act, x, d, L.ln1_w, L.ln1_b, rows, d, kLnEps, e->xn.p, d, s));
     // q | k | v: rd(rd(h W^T) + b), q and k then rd(. * rd(head_dim^-1/4))
     GemmArgs g = gemm(e->xn.p, d, L.qkv, rows, e->qkv.p, 3 * d);
     g.aff.bias = L.qkv_b;
@@ -188,27 +192,23 @@ int run_layers(fmd_enc* e, int windows, int t, int first, int n, bool final_norm
     // x = rd(x + rd(rd(ctx Wo^T) + bo))
     g = gemm(e->ctx.p, d, L.o, rows, e->x.p, d);
     g.aff.bias = L.o_b;
-    g.resid = e->x.p;
+    g.resid = x;
     LAUNCH(launch_gemm(act, EPI_AFFINE, g, s));
-    LAUNCH(launch_layernorm(act, e->x.p, d, L.ln2_w, L.ln2_b, rows, d, kLnEps, e->xn.p, d, s));
+    x = e->x.p;
+    LAUNCH(launch_layernorm(act, x, d, L.ln2_w, L.ln2_b, rows, d, kLnEps, e->xn.p, d, s));
     g = gemm(e->xn.p, d, L.fc1, rows, e->ff.p, e->f);
     g.aff.bias = L.fc1_b;
     g.aff.act = 1;
     LAUNCH(launch_gemm(act, EPI_AFFINE, g, s));
-    g = gemm(e->ff.p, e->f, L.fc2, rows, e->x.p, d);
+    g = gemm(e->ff.p, e->f, L.fc2, rows, l + 1 == first + n && !final_norm ? out : e->x.p, d);
     g.aff.bias = L.fc2_b;
-    g.resid = e->x.p;
+    g.resid = x;
     LAUNCH(launch_gemm(act, EPI_AFFINE, g, s));
   }
-  const size_t es = e->esz;
-  if (final_norm) {
-    LAUNCH(launch_layernorm(act, e->x.p, d, e->ln_w, e->ln_b, rows, d, kLnEps, e->xn.p, d, s));
-    HIPCHK(hipMemcpy2DAsync(out, (size_t)t * d * es, e->xn.p, (size_t)P * d * es,
-                            (size_t)t * d * es, windows, hipMemcpyDeviceToDevice, s));
-  } else {
-    HIPCHK(hipMemcpy2DAsync(out, (size_t)t * d * es, e->x.p, (size_t)P * d * es,
-                            (size_t)t * d * es, windows, hipMemcpyDeviceToDevice, s));
-  }
+  if (final_norm)
+    LAUNCH(launch_layernorm(act, x, d, e->ln_w, e->ln_b, rows, d, kLnEps, out, d, s));
+  else if (n == 0 && out != in)
+    HIPCHK(hipMemcpyAsync(out, in, (size_t)rows * d * e->esz, hipMemcpyDeviceToDevice, s));
   return 0;
 }
 
@@ -244,7 +244,11 @@ int forward_windows(fmd_enc* e, const void* mel_dev, int mel_dtype, int windows,
   g.aff.period = P;
   g.aff.valid = t;
   LAUNCH(launch_gemm(act, EPI_AFFINE, g, s));
-  return run_layers(e, windows, t, 0, (int)e->layers.size(), true, out);
+  CHK(run_layers(e, windows, t, P, 0, (int)e->layers.size(), true, e->x.p, e->xn.p));
+  // without the spare row after each window
+  HIPCHK(hipMemcpy2DAsync(out, (size_t)t * d * es, e->xn.p, (size_t)P * d * es, (size_t)t * d * es, windows,
+                          hipMemcpyDeviceToDevice, s));
+  return 0;
 }
 
 int check_frames(const fmd_enc* e, int frames) {
@@ -524,15 +528,22 @@ extern "C" int fmd_enc_layers(fmd_enc* e, const void* x, int x_on_device, int wi
   const size_t es = e->esz, row = (size_t)e->d * es, bytes = (size_t)windows * t * row;
   const void* src = nullptr;
   CHK(stage(e, e->hin, x, bytes, x_on_device, &src));
-  // into the (t + 1)-row window layout
-  HIPCHK(hipMemcpy2DAsync(e->x.p, (size_t)(t + 1) * row, src, (size_t)t * row, (size_t)t * row,
-                          windows, hipMemcpyDeviceToDevice, e->stream));
   void* dst = out;
-  if (!out_on_device) {
+  if (!out_on_device || (uintptr_t)out % 16) {
     CHK(e->frames.ensure(bytes));
     dst = e->frames.p;
   }
-  CHK(run_layers(e, windows, t, first, n, final_norm != 0, dst));
+  // through e->x where the kernels' 16-byte accesses do not allow the caller's
+  // rows, and without layers, whose output may overlap them
+  if ((uintptr_t)src % 16 || n == 0) {
+    HIPCHK(hipMemcpyAsync(e->x.p, src, bytes, hipMemcpyDeviceToDevice, e->stream));
+    src = e->x.p;
+  }
+  // the windows without spare rows (only conv2 needs those): no copies in or
+  // out around the layers
+  CHK(run_layers(e, windows, t, t, first, n, final_norm != 0, src, dst));
+  if (out_on_device && dst != out)
+    HIPCHK(hipMemcpyAsync(out, dst, bytes, hipMemcpyDeviceToDevice, e->stream));
   if (!out_on_device) HIPCHK(hipMemcpyAsync(out, dst, bytes, hipMemcpyDeviceToHost, e->stream));
   HIPCHK(hipStreamSynchronize(e->stream));
   return 0;

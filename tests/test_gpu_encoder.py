@@ -297,3 +297,31 @@ def test_attention_key_blocks_and_growing_scores(fmd, orc, t, windows):
     for i in (0, windows - 1):
         alone = gpu.layers(from_f32(x[i:i + 1], "f16", orc), 0, 1)
         assert np.array_equal(alone[0], got[i]), i
+
+
+@pytest.mark.parametrize("n,final_norm", [(0, 0), (0, 1), (1, 0), (2, 0), (2, 1)])
+def test_layers_on_device_buffers(fmd, n, final_norm):
+    """fmd_enc_layers on device rows gives the bits of the host call: into
+    another buffer (the input is left as it was), in place, into a buffer that
+    overlaps the input, and for rows that are not 16-byte aligned."""
+    import torch
+
+    print(f"[gpu] encoder layers on device n={n} norm={final_norm}", flush=True)
+    cfg = acfg(fmd, layers=2)
+    gpu = fmd.AudioEncoder(cfg, "bf16").load(fmd.synthetic_audio_weights(cfg, seed=23))
+    W, t, d = 3, 37, cfg.d_model
+    x = torch.randn((W, t, d), generator=torch.Generator().manual_seed(24)).bfloat16()
+    want = torch.from_numpy(gpu.layers(x.view(torch.int16).numpy().view(np.uint16), 0, n, bool(final_norm)).view(np.int16))
+    size, lib = W * t * d, fmd.lib()
+    for xo, yo in ((0, size + 8), (0, 0), (0, 8 * d), (8 * d, 0), (1, size + 9), (0, size + 9), (1, size + 16)):
+        buf = torch.zeros(2 * size + 32, dtype=torch.int16, device="cuda")
+        buf[xo:xo + size] = x.view(torch.int16).reshape(-1).cuda()
+        before = buf.clone()
+        torch.cuda.synchronize()
+        rc = lib.fmd_enc_layers(gpu.handle, buf.data_ptr() + 2 * xo, 1, W, t, 0, n, final_norm,
+                                buf.data_ptr() + 2 * yo, 1)
+        assert rc == 0, lib.fmd_last_error()
+        torch.cuda.synchronize()
+        assert torch.equal(buf[yo:yo + size].cpu().reshape(W, t, d), want), (xo, yo)
+        before[yo:yo + size] = buf[yo:yo + size]
+        assert torch.equal(before, buf), (xo, yo)
