@@ -163,7 +163,8 @@ int fmd_dec_assemble(fmd_dec* dec, const uint32_t* ids, const int64_t* offsets, 
  * (batch, total, hidden) left-padded in the activation dtype (host, or device
  * when embeds_on_device); pad[b] = left padding of row b.  Queries are taken
  * `chunk` positions at a time (the reference uses 256; pad rows are exactly
- * zero in the reference and are skipped).  Writes f32 logits (batch, vocab)
+ * zero in the reference and are skipped), and more while those hold fewer than
+ * 12,288 real rows.  Writes f32 logits (batch, vocab)
  * of each row's last position to `logits` (host) when non-NULL.  The cache
  * must be empty; its length becomes `total`. */
 int fmd_dec_prefill(fmd_dec* dec, fmd_kv* kv, const void* embeds, int embeds_on_device,

@@ -266,6 +266,38 @@ def test_layer_decode_on_unaligned_rows_and_moved_lengths(fmd, prec, B):
     assert kv.len() == 100
 
 
+@pytest.mark.parametrize("prec,lens,chunk", [
+    ("f16", (3000, 1, 1100, 2500) + (900,) * 8, 64),     # 13,801 rows: two chunks
+    ("int8", (2049,) * 6, 256),                          # one chunk of 12,288 rows and one of 6
+    ("bf16", (3300, 1000, 3300, 200, 3299, 3300), 2000), # `chunk` positions hold more at the end
+])
+def test_prefill_chunks_by_rows(fmd, orc, prec, lens, chunk):
+    """Chunks take `chunk` positions or 12,288 real rows, whichever is more:
+    left padding, rows that begin inside a chunk, and a last chunk of a few
+    rows.  Logits and both layers' caches against the oracle."""
+    _announce(f"prefill chunks by rows {prec} {lens} chunk={chunk}")
+    cfg = tiny_cfg(fmd)
+    gpu, ref, _ = build_pair(fmd, orc, cfg, prec, seed=40, max_len=3400)
+    rng = np.random.default_rng(sum(lens))
+    emb, pad = ref.padded_embeds([rng.integers(0, cfg.vocab_size, n).tolist() for n in lens])
+    T = max(lens)
+    gkv, rkv = gpu.new_caches(len(lens), T + 4), ref.new_kv(len(lens), T + 4)
+    got = gpu.prefill(orc.to_storage(emb, OPREC[prec]), gkv, pad, chunk=chunk)
+    want = ref.prefill(rkv, emb, pad, block=256)
+    assert np.max(np.abs(got - want)) < TOL[prec]
+    for layer in range(2):
+        for which in (0, 1):
+            g, r = storage_to_f32(gkv.read(layer, which), prec), rkv.read(layer, which)
+            for b, n in enumerate(lens):
+                p = T - n
+                assert not g[b, :, :p].any() and not g[b, :, T:].any(), (layer, which, b)
+                d = g[b, :, p:T] - r[b, :, p:T]
+                assert np.linalg.norm(d) <= 1e-2 * np.linalg.norm(r[b, :, p:T]), (layer, which, b)
+    # a whole call twice on one cache gives the same bits
+    gkv.truncate(0)
+    assert np.array_equal(gpu.prefill(orc.to_storage(emb, OPREC[prec]), gkv, pad, chunk=chunk), got)
+
+
 # --------------------------------------------------------------------------
 # decode step over a synthetic padded context (configs 2 / 3 style)
 # --------------------------------------------------------------------------
