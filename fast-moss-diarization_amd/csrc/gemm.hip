@@ -5,9 +5,9 @@
 // 16x32 fragment):
 // - small grids (gemm_small_kernel): tiles of 32 to 128 rows x 32 to 128
 //   columns, dense or Q8_0, chosen so that the grid covers the CUs (try_small);
-// - dense 16-bit weights (gemm_dma_kernel, 64, 128 or 256 rows x 128 columns):
+// - dense 16-bit weights (gemm_dma_kernel, 128 or 256 rows x 128 columns):
 //   both operands go global -> LDS by direct-to-LDS loads through a ring of
-//   32-k stages; waves hold 32 x 64, 64 x 64 or 128 x 64;
+//   32-k stages; waves hold 64 x 64 or 128 x 64;
 // - Q8_0 (gemm_q8_kernel, 64 rows x 128 columns): K step 64, X staged global ->
 //   registers -> LDS, double-buffered with one barrier per K step (row pitch
 //   padded to 72 elements so the MFMA-order 16-byte reads are bank-conflict
@@ -562,14 +562,14 @@ gemm_q8_kernel(GemmArgs p) {
 // 16-bit activations with dense 16-bit weights, both operands copied global
 // -> LDS by the direct-to-LDS loads (no register staging): a ring of NS
 // stages of BK2 = 32 k, NS - 1 steps in flight, one barrier per step.  Tile
-// BMT x 128 (BMT 64, 128 or 256), four waves of BMT/2 x 64 (same fragments and
+// BMT x 128 (BMT 128 or 256), four waves of BMT/2 x 64 (same fragments and
 // XCD work order as gemm_q8_kernel).  X stage: BMT rows x 4
 // chunks of 8 elements, chunk c of row r at slot r * 4 + (c ^ swz(r)), so
 // that the fragment reads of any 8 consecutive lanes fall in distinct
 // 16-byte bank groups of 128 bytes and those of any 16 in distinct groups of
 // 256 bytes; W stage: the work-group's 8 weight tiles, each one 1 KiB
 // fragment of the tiled layout.  LDS: NS * (BMT * 64 + 8192) bytes, so two
-// work-groups per CU at (128, 4) and (256, 3), three at (64, 4).
+// work-groups per CU at (128, 4) and (256, 3).
 constexpr int BK2 = 32;
 
 __device__ __forceinline__ int swz(int r) { return ((r >> 1) ^ (r >> 3)) & 3; }
@@ -816,7 +816,7 @@ template <int A, int EPI, int BMT, int NS>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2)))
 gemm_dma_kernel(GemmArgs p) {
   typedef typename ActT<A>::T T;
-  static_assert(((BMT == 64 || BMT == 128) && NS == 4) || (BMT == 256 && NS == 3), "tile / ring");
+  static_assert((BMT == 128 && NS == 4) || (BMT == 256 && NS == 3), "tile / ring");
   constexpr int MI = BMT / 32;           // 16-row fragments per wave
   constexpr int NX = BMT / 64;           // X copies per thread per stage
   constexpr int PER = NX + 2;            // copies per thread per stage
@@ -846,7 +846,7 @@ gemm_dma_kernel(GemmArgs p) {
   }
   const int mb = m0 + wm * (BMT / 2);
   [[maybe_unused]] uint2 rres[MI][4];   // in flight behind the K loop
-  static_assert(EPI != EPI_RESID || BMT <= 128, "residual prefetch: 64- and 128-row tiles");
+  static_assert(EPI != EPI_RESID || BMT <= 128, "residual prefetch: 128-row tiles");
   if constexpr (EPI == EPI_RESID) cross_resid<true, MI, 4>(p, mb, tile, tv, rres);
   // This thread's copies per stage: X slots j * 64 + lane of instructions
   // j = NX w .. NX w + NX - 1 (rows 16 j + lane / 4; rows past M read row
@@ -1246,23 +1246,19 @@ __global__ void __launch_bounds__(256) gemm32_kernel(GemmArgs p) {
   }
 }
 
-// Tile of the 16-bit dense products past the small grids (512 work-groups =
-// two per CU), chosen from bf16 sweeps over the prefill shapes and row counts:
-// - 256 rows where 256-row tiles fill at least 7/8 of the slots and do not end
-//   in a last round of fewer than 128 work-groups (qkv M = 3584 36.5 against
-//   38.9 us, M = 4096 39.2 against 42.4; gate|up M = 2560 38.0 against 41.4,
-//   M = 4096 59.8 against 62.9, but M = 3072, 576 tiles, 56.2 against 51.9);
-// - 128 rows where their grid fills the slots, and for wide outputs (16 or more
-//   column groups) also below that (qkv M = 1328 19.5 against 22.3 us for
-//   64-row tiles, M = 1560 20.9 against 27.6);
-// - narrow outputs otherwise take 64 rows.
-enum GemmTile { TILE64, TILE128, TILE256 };
-GemmTile gemm_tile(int M, int col_groups) {
-  const int tiles128 = (M + 127) / 128 * col_groups;
+// Rows of the 16-bit dense tiles past the small grids (512 work-groups = two
+// per CU), chosen from bf16 sweeps over the prefill shapes and row counts: 256
+// where those tiles fill about 4/5 of the slots and do not end in a last round
+// of fewer than 128 work-groups (qkv M = 3584 36.5 against 38.9 us, M = 4096
+// 39.2 against 42.4; down M = 13509, 424 tiles, 95.5 against 108.6, but M =
+// 12008, 376 tiles, 90.2 against 86.1; gate|up M = 2560 38.0 against 41.4, but
+// M = 3072, 576 tiles, 56.2 against 51.9), else 128 (64-row tiles, which
+// narrow outputs took up to 512 tiles of 128 rows, were slower past the small
+// grids: O M = 4503 33.8 against 31.3 us, M = 7505 44.8 against 37.0; down
+// 47.7 against 43.3 and 66.2 against 53.3).
+int gemm_tile_rows(int M, int col_groups) {
   const int tiles256 = (M + 255) / 256 * col_groups;
-  if (tiles256 >= 448 && (tiles256 % 512 == 0 || tiles256 % 512 >= 128)) return TILE256;
-  if (tiles128 >= 512 || col_groups >= 16) return TILE128;
-  return TILE64;
+  return tiles256 >= 400 && (tiles256 % 512 == 0 || tiles256 % 512 >= 128) ? 256 : 128;
 }
 
 // Whether the dense tiles may move 16 bytes of output, bias, residual and table
@@ -1417,22 +1413,18 @@ hipError_t dispatch(int epi, const GemmArgs& a, hipStream_t s) {
       hipError_t e = hipSuccess;
       if (try_small<A, WK>(epi, a, s, &e)) return e;
     }
-    GemmTile tt = WK == WK_Q8 ? TILE64 : gemm_tile(a.M, cols);
+    int bm = WK == WK_Q8 ? 64 : gemm_tile_rows(a.M, cols);
     // the fused q/k norm + RoPE epilogue stages at most 128 rows (a 256-row
     // tile would spill), and the residuals a 256-row tile would prefetch do
     // not fit its registers: 128-row tiles instead
-    if ((epi == EPI_ROPE || epi == EPI_RESID) && tt == TILE256) tt = TILE128;
-    const int bm = tt == TILE256 ? 256 : tt == TILE128 ? 128 : 64;
+    if ((epi == EPI_ROPE || epi == EPI_RESID) && bm == 256) bm = 128;
     GemmArgs g = a;
     g.map = xcd_rows(a, cols, bm);
     const int mtiles = (a.M + bm - 1) / bm, Ma = (mtiles + g.map - 1) / g.map;
     const dim3 grid(8 * Ma * (cols / (8 / g.map)));
     if constexpr (WK == WK_Q8) return launch_q8(epi, grid, g, s);
-    else {
-      if (tt == TILE256) return launch_dma<A, 256, 3>(epi, grid, g, s);
-      if (tt == TILE128) return launch_dma<A, 128, 4>(epi, grid, g, s);
-      return launch_dma<A, 64, 4>(epi, grid, g, s);
-    }
+    else if (bm == 256) return launch_dma<A, 256, 3>(epi, grid, g, s);
+    else return launch_dma<A, 128, 4>(epi, grid, g, s);
   }
 }
 
