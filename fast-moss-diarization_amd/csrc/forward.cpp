@@ -642,8 +642,15 @@ int prefill_impl(fmd_dec* d, fmd_kv* kv, const void* emb_dev, const int32_t* pad
       long blocks = 0;
       for (int t = 0; t < nt; ++t)
         blocks += (tiles[2 * maxTiles + t] + tiles[3 * maxTiles + t] - pad[tiles[t]] + 63) / 64;
-      // items per tile <= its blocks / split_blocks + 1, so nitems <= nt + kItemsPerHead
-      const long split_blocks = std::max(4L, (blocks + kItemsPerHead - 1) / kItemsPerHead);
+      // items per tile <= its blocks / split_blocks + 1, so nitems <= nt + kItemsPerHead.
+      // The f16 kernel passes over its keys once, so its pieces are half as
+      // many and not under 12 blocks, which saves merging (a two-layer prefill
+      // at >= 4 blocks and 192 pieces | 12 and 96: four prompts of 310-1890
+      // 694 | 672 us, eight of 300-1200 1064 | 1034, eight of 2000-5000 3691 |
+      // 3590; one of 450 or 1000 within noise).
+      const bool one_pass = act == ACT_F16;
+      const long pieces = one_pass ? kItemsPerHead / 2 : kItemsPerHead;
+      const long split_blocks = std::max(one_pass ? 12L : 4L, (blocks + pieces - 1) / pieces);
       const int split = (int)(64 * split_blocks);
       int32_t* t_first = tiles + 4 * maxTiles;
       int32_t* t_ns = tiles + 5 * maxTiles;
