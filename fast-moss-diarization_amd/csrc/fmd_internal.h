@@ -50,12 +50,12 @@ struct DecodeLane {
 // Per-handle device scratch, sized on demand (never inside a graph capture).
 struct Workspace {
   DevBuf x, xn, qkv, q, ctx, act, logits, amax, pml, po, ids, pad, rowmeta, tiles, lastx, embeds,
-      done, ntok, finish, tokens, force, opstate, oppad, asrc, audio;
+      done, ntok, finish, tokens, force, gstate, opstate, oppad, asrc, audio;
   DecodeLane dec;
   void release_all() {
     for (DevBuf* b : {&x, &xn, &qkv, &q, &ctx, &act, &logits, &amax, &pml, &po, &ids, &pad,
                       &rowmeta, &tiles, &lastx, &embeds, &done, &ntok, &finish, &tokens, &force,
-                      &opstate, &oppad, &asrc, &audio})
+                      &gstate, &opstate, &oppad, &asrc, &audio})
       b->release();
     dec.release_all();
   }
@@ -81,7 +81,8 @@ struct fmd_dec {
   int32_t* host_mirror = nullptr;  // host-mapped copy of the greedy state and the attention error code
   void* host_stage = nullptr;      // pinned host staging of prefill chunk tables
   size_t host_stage_n = 0;
-  // what fmd_op_attention_decode last uploaded (repeated calls skip the copies)
+  // what fmd_op_attention_decode last uploaded to ws.opstate and ws.oppad, which
+  // only it writes (repeated calls skip the copies)
   std::vector<int32_t> op_pad;
   int op_len = -1;
   int logits_rows = 0;  // rows of the last logits launch (prefill / decode step), 0 = none

@@ -1045,6 +1045,7 @@ extern "C" int fmd_op_attention_decode(fmd_dec* d, fmd_kv* kv, int layer, const 
   const std::vector<int32_t> padv(pad, pad + B);
   if (d->op_len != kv->len || d->op_pad != padv || d->op_state_buf != w.opstate.p ||
       d->op_pad_buf != w.oppad.p) {
+    d->op_len = -1;   // not what is there until both copies are issued
     int32_t st[4] = {kv->len, 0, 0, 0};
     HIPCHK(hipMemcpyAsync(w.opstate.p, st, sizeof st, hipMemcpyHostToDevice, d->stream));
     HIPCHK(hipMemcpyAsync(w.oppad.p, pad, (size_t)B * 4, hipMemcpyHostToDevice, d->stream));
@@ -1080,14 +1081,14 @@ extern "C" int fmd_dec_greedy(fmd_dec* d, int B, uint32_t eos, const int32_t* fo
   CHK(w.finish.ensure((size_t)B * 4));
   CHK(w.tokens.ensure((size_t)B * 4));
   CHK(w.force.ensure((size_t)B * 4));
-  CHK(w.opstate.ensure(64));
+  CHK(w.gstate.ensure(64));
   CHK(w.ids.ensure((size_t)B * 4));
   CHK(w.x.ensure((size_t)B * d->H * d->esz));
   hipStream_t s = d->stream;
   // one greedy update with a token budget of 1: ntok[b] tells whether row b
   // emitted a token this step
   const int32_t st[4] = {0, step, 0, 0};
-  HIPCHK(hipMemcpyAsync(w.opstate.p, st, sizeof st, hipMemcpyHostToDevice, s));
+  HIPCHK(hipMemcpyAsync(w.gstate.p, st, sizeof st, hipMemcpyHostToDevice, s));
   HIPCHK(hipMemcpyAsync(w.done.p, done, (size_t)B * 4, hipMemcpyHostToDevice, s));
   HIPCHK(hipMemsetAsync(w.ntok.p, 0, (size_t)B * 4, s));
   HIPCHK(hipMemsetAsync(w.finish.p, 0, (size_t)B * 4, s));
@@ -1096,7 +1097,7 @@ extern "C" int fmd_dec_greedy(fmd_dec* d, int B, uint32_t eos, const int32_t* fo
   g.part = w.amax.as<uint64_t>();
   g.nparts = gemv_logits_nparts(d->act, d->quant, true, d->H, d->V);
   g.batch = B;
-  g.state = w.opstate.as<int32_t>();
+  g.state = w.gstate.as<int32_t>();
   g.host_state = nullptr;
   g.advance = 0;
   g.done = w.done.as<int32_t>();

@@ -472,6 +472,35 @@ def test_attention_exchange_buffers_regrow_across_handles(fmd, orc):
         del gpu, kv
 
 
+def test_attention_decode_after_a_greedy_update(fmd):
+    """fmd_op_attention_decode uploads the write position and the pads only when
+    they changed: a greedy update between two calls with the same ones does not
+    disturb them (context, the appended key's position, and the cache's other
+    positions)."""
+    _announce("attention decode, greedy, attention decode")
+    cfg = tiny_cfg(fmd, layers=1)
+    gpu = fmd.Qwen3(cfg, "int8", max_len=512).load(fmd.synthetic_weights(cfg, seed=41))
+    B, L = 2, 300
+    kv, other = gpu.new_caches(B, 320), gpu.new_caches(B, 8)
+    kv.fill_random(6, L)
+    gpu.prefill(np.ones((B, 4, cfg.hidden_size), np.float16), other, [0, 1])
+    qkv = torch.randn((B, cfg.q_dim() + 2 * cfg.kv_dim()), generator=torch.Generator().manual_seed(42))
+    qkv = qkv.half().cuda()
+    outs, caches = [], []
+    for step in range(3):
+        out = torch.empty(B, cfg.q_dim(), dtype=torch.float16, device="cuda")
+        torch.cuda.synchronize()
+        gpu.op_attention_decode(kv, 0, qkv.data_ptr(), [0, 7], B, out.data_ptr())
+        torch.cuda.synchronize()
+        outs.append(out)
+        caches.append([kv.read(0, which) for which in (0, 1)])
+        gpu.greedy(B, step, np.zeros(B, dtype=np.int32), eos=5)
+    for out, cache in zip(outs[1:], caches[1:]):
+        assert torch.equal(out, outs[0])
+        for a, b in zip(cache, caches[0]):
+            assert np.array_equal(a, b)
+
+
 # --------------------------------------------------------------------------
 # prefill + KV-cache contents
 # --------------------------------------------------------------------------
