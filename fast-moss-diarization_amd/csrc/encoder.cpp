@@ -560,6 +560,13 @@ extern "C" int fmd_enc_adaptor(fmd_enc* e, const void* frames, int frames_on_dev
   const size_t es = e->esz;
   const void* src = nullptr;
   CHK(stage(e, e->joined, frames, (size_t)g * e->ain * es, frames_on_device, &src));
+  if ((uintptr_t)src % 16) {
+    // the products' direct-to-LDS copies read 16 aligned bytes
+    const size_t bytes = (size_t)g * e->ain * es;
+    CHK(e->joined.ensure(bytes));
+    HIPCHK(hipMemcpyAsync(e->joined.p, src, bytes, hipMemcpyDeviceToDevice, e->stream));
+    src = e->joined.p;
+  }
   void* dst = out;
   if (!out_on_device) {
     CHK(e->aout.ensure((size_t)g * e->H * es));

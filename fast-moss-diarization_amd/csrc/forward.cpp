@@ -1013,6 +1013,13 @@ extern "C" int fmd_op_linear(fmd_dec* d, int layer, int proj, const void* x, int
                          gemv_args(xs, in, nullptr, d->eps, l->w, n, ys, out, nullptr, nullptr),
                          d->stream));
     } else {
+      if (d->act != ACT_F32 && (uintptr_t)xs % 16) {
+        // the tiles' direct-to-LDS copies read 16 aligned bytes
+        const size_t bytes = (size_t)n * in * d->esz;
+        CHK(d->ws.xn.ensure(bytes));
+        HIPCHK(hipMemcpyAsync(d->ws.xn.p, xs, bytes, hipMemcpyDeviceToDevice, d->stream));
+        xs = d->ws.xn.as<char>();
+      }
       GemmArgs g{};
       g.x = xs;
       g.ldx = in;

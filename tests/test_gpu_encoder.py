@@ -207,6 +207,37 @@ def test_adaptor_full_window(fmd, orc, dt):
     assert gpu.merge_and_project(from_f32(frames[:7], dt, orc)).shape == (1, 1024)
 
 
+@pytest.mark.parametrize("dt", ["f16", "bf16"])
+@pytest.mark.parametrize("rows", [5, 1500, 13000])
+def test_adaptor_on_device_rows_of_any_alignment(fmd, dt, rows):
+    """fmd_enc_adaptor on device frames that begin on any element gives the bits
+    of the host call (rows of one merged group, of a window, and past the small
+    grids), and leaves the frames as they were."""
+    import torch
+
+    print(f"[gpu] adaptor rows of any alignment {dt} rows={rows}", flush=True)
+    cfg = full(fmd, 0)
+    gpu = fmd.AudioEncoder(cfg, "int8" if dt == "f16" else dt).load(fmd.synthetic_audio_weights(cfg, seed=25))
+    tdt = torch.float16 if dt == "f16" else torch.bfloat16
+    x = torch.randn((rows, 1024), generator=torch.Generator().manual_seed(26)).to(tdt)
+    host = x.view(torch.int16).numpy().view(np.uint16) if dt == "bf16" else x.numpy()
+    want = gpu.merge_and_project(host)
+    out = torch.empty(want.shape, dtype=tdt, device="cuda")
+    for off in (0, 1):
+        buf = torch.zeros(rows * 1024 + 8, dtype=tdt, device="cuda")
+        buf[off:off + rows * 1024] = x.reshape(-1).cuda()
+        before = buf.clone()
+        torch.cuda.synchronize()
+        rc = fmd.lib().fmd_enc_adaptor(gpu.handle, buf.data_ptr() + off * buf.element_size(), 1, rows,
+                                       out.data_ptr(), 1)
+        assert rc == 0, fmd.lib().fmd_last_error()
+        torch.cuda.synchronize()
+        got = out.cpu()
+        got = got.view(torch.int16).numpy().view(np.uint16) if dt == "bf16" else got.numpy()
+        assert np.array_equal(got, want), off
+        assert torch.equal(buf, before), off
+
+
 @pytest.mark.parametrize("dt", ["f32", "bf16"])
 def test_encode_audio_reassembly(fmd, orc, dt):
     """mod.rs:82-126 over five chunks of three audios: each chunk trimmed to

@@ -193,6 +193,27 @@ def test_linear_tile_kinds_give_the_same_bits(fmd, prec):
             assert not buf[:1].any() and not buf[1 + m * n:].any()
 
 
+@pytest.mark.parametrize("prec", ["f16", "bf16", "int8"])
+def test_linear_rows_of_any_alignment(fmd, prec):
+    """Rows that begin on any element give the bits of aligned rows, in the
+    small-grid tiles (17 and 300 rows) and the tiles past them (4300)."""
+    _announce(f"linear rows of any alignment {prec}")
+    cfg = small_cfg(fmd, layers=1, vocab=256)
+    gpu = fmd.Qwen3(cfg, prec, max_len=64).load(fmd.synthetic_weights(cfg, seed=43))
+    dt = torch.bfloat16 if prec == "bf16" else torch.float16
+    for proj, (k, n) in {0: (1024, 4096), 3: (3072, 1024)}.items():
+        x = torch.randn((4300, k), generator=torch.Generator().manual_seed(proj)).to(dt).cuda()
+        for m in (17, 300, 4300):
+            want, got = (torch.empty((m, n), dtype=dt, device="cuda") for _ in range(2))
+            buf = torch.zeros(m * k + 8, dtype=dt, device="cuda")
+            buf[1:1 + m * k] = x[:m].reshape(-1)
+            torch.cuda.synchronize()
+            gpu.op_linear(0, proj, x.data_ptr(), m, want.data_ptr())
+            gpu.op_linear(0, proj, buf.data_ptr() + buf.element_size(), m, got.data_ptr())
+            torch.cuda.synchronize()
+            assert torch.equal(got, want), (proj, m)
+
+
 @pytest.mark.parametrize("prec,n", [("int8", 20), ("int8", 225), ("int8", 450), ("f16", 65),
                                     ("bf16", 257), ("bf16", 700)])
 def test_prefill_small_grids_full_width(fmd, orc, prec, n):
