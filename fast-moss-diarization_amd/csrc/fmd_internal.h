@@ -92,6 +92,9 @@ struct fmd_dec {
   // the call fails (fmd_dec_set_spin_limit); each poll is a device-memory
   // round trip, about a microsecond.
   int spin_limit = 20000;
+  // Real rows that a prefill chunk is filled up to past its `chunk` positions
+  // (fmd_dec_set_prefill_rows; chunk_positions has the figures).
+  int prefill_rows = 12288;
   // Device seconds of the prefills and the greedy decode loops run by
   // fmd_dec_generate since the last reset (HIP events around each part).
   double t_prefill = 0.0, t_decode = 0.0;

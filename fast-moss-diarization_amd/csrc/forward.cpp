@@ -499,33 +499,37 @@ extern "C" int fmd_dec_assemble(fmd_dec* d, const uint32_t* ids, const int64_t* 
 namespace {
 
 // Positions that a prefill chunk from `start` takes: `chunk` of them, and more
-// while they hold fewer than kChunkRows real (non-pad) rows.  Left-padded
-// batches have few rows in their first positions, small or short batches in all
-// of them, and a layer's launches on few rows cost their latency, an unfilled
-// last round of tiles, or attention items too short to be worth merging.
+// while they hold fewer than `fill` real (non-pad) rows (fmd_dec::prefill_rows).
+// Left-padded batches have few rows in their first positions, small or short
+// batches in all of them, and a layer's launches on few rows cost their latency,
+// an unfilled last round of tiles, or attention items too short to be worth
+// merging.
 // Two layers, us a prefill at 512 | 2048 | 4096 | 8192 | 12288 | 16384 rows:
 //   one prompt of 3000, bf16            1276 |   860 |   722 |   725 |   723 |   736
 //   four of 310-1890, f16, chunk 256    1113 |   833 |   682 |   684 |   692 |   701
 //   eight of 300-1200, int8, chunk 256  1623 |  1382 |  1250 |  1039 |  1024 |  1034
 //   eight of 500-4000, bf16, chunk 256  4361 |  3677 |  2892 |  2479 |  2350 |  2155
 //   eight of 1500-8000, bf16, chunk 512    - |     - | 12372 | 11120 | 10312 | 10300
-// (at 12288 rows of the 0.6B shape the activations take 0.4 GB and the attention's
-// split results 0.2 GB).  Which rows share a chunk changes no row's products,
-// and its attention only in where the keys are cut into items.
-constexpr int kChunkRows = 12288;
-
-int chunk_positions(const int32_t* pad, int B, int start, int total, int chunk) {
+// 12288 is the default: no case but the fourth gains from more, its workspace is
+// three quarters of 16384's (12288 rows of the 0.6B shape: activations 0.4 GB,
+// the attention's split results 0.2 GB), and the bf16 logits of the last case
+// stay within their bar, which other row counts straddle (largest difference
+// from the reference's rounding, bar 0.02: 2048 .0215, 4096 .0176, 8192 .0234,
+// 12288 .0195, 16384 .0215; rms .0049 at each).
+// Which rows share a chunk changes no row's products, and its attention only in
+// where the keys are cut into items.
+int chunk_positions(const int32_t* pad, int B, int start, int total, int chunk, int fill) {
   int end = start + std::min(chunk, total - start);
   int64_t rows = 0;
   for (int b = 0; b < B; ++b) rows += std::max(0, end - std::max(start, (int)pad[b]));
-  while (end < total && rows < kChunkRows) {
+  while (end < total && rows < fill) {
     // up to where another row begins, or the missing rows are there
     int active = 0, next = total;
     for (int b = 0; b < B; ++b) {
       if (pad[b] <= end) ++active;
       else next = std::min(next, (int)pad[b]);
     }
-    const int64_t want = active ? (kChunkRows - rows + active - 1) / active : next - end;
+    const int64_t want = active ? (fill - rows + active - 1) / active : next - end;
     const int step = (int)std::min<int64_t>(want, next - end);
     end += step;
     rows += (int64_t)step * active;
@@ -542,8 +546,10 @@ int prefill_impl(fmd_dec* d, fmd_kv* kv, const void* emb_dev, const int32_t* pad
   const int act = d->act;
   const int QT = attn_prefill_tile_rows(d->rep);
   // rows of a chunk (chunk_positions): B per position, or past `chunk`
-  // positions fewer than B more than kChunkRows
-  const int maxM = (int)std::min<int64_t>((int64_t)B * total, std::max<int64_t>((int64_t)B * chunk, kChunkRows + B));
+  // positions fewer than B more than `fill`
+  const int fill = d->prefill_rows;
+  const int maxM =
+      (int)std::min<int64_t>((int64_t)B * total, std::max<int64_t>((int64_t)B * chunk, (int64_t)fill + B));
   CHK(ensure_decode_ws(d, std::min(B, kMaxDecodeRows), kv->cap));
   CHK(w.x.ensure((size_t)(maxM + 1) * d->H * d->esz));
   CHK(w.xn.ensure((size_t)maxM * std::max(d->H, d->I) * d->esz));
@@ -606,7 +612,7 @@ int prefill_impl(fmd_dec* d, fmd_kv* kv, const void* emb_dev, const int32_t* pad
   const int32_t* dtiles = w.tiles.as<int32_t>();
 
   for (int start = 0, c = 0, len = 0; start < total; start += len, ++c) {
-    len = chunk_positions(pad, B, start, total, chunk);
+    len = chunk_positions(pad, B, start, total, chunk, fill);
     if (c >= 2) HIPCHK(hipEventSynchronize(stage.ev[c & 1]));
     int32_t* meta = (int32_t*)d->host_stage + (size_t)(c & 1) * (meta_n + tiles_n);
     int32_t* tiles = meta + meta_n;
@@ -1136,6 +1142,13 @@ extern "C" int fmd_dec_set_spin_limit(fmd_dec* d, int polls) {
   if (!d) return fmd_fail(FMD_ERR_ARG, "null handle");
   if (polls < 0) return fmd_fail(FMD_ERR_ARG, "negative poll count");
   d->spin_limit = polls;
+  return 0;
+}
+
+extern "C" int fmd_dec_set_prefill_rows(fmd_dec* d, int rows) {
+  if (!d) return fmd_fail(FMD_ERR_ARG, "null handle");
+  if (rows < 0) return fmd_fail(FMD_ERR_ARG, "negative row count");
+  d->prefill_rows = rows;
   return 0;
 }
 

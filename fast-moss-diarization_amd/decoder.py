@@ -95,6 +95,7 @@ SIGNATURES = {
     "fmd_dec_destroy": (_I, [_P]),
     "fmd_dec_set_stream": (_I, [_P, _P]),
     "fmd_dec_set_spin_limit": (_I, [_P, _I]),
+    "fmd_dec_set_prefill_rows": (_I, [_P, _I]),
     "fmd_dec_stream": (_P, [_P]),
     "fmd_dec_set_weight": (_I, [_P, ctypes.c_char_p, _I, ctypes.POINTER(_I64), _I, _P, _I]),
     "fmd_dec_ready": (_I, [_P]),
@@ -604,6 +605,11 @@ class Qwen3:
     def set_spin_limit(self, polls: int) -> None:
         """Polls before a wait of the decode attention gives up (the call then fails)."""
         _check(lib().fmd_dec_set_spin_limit(self.handle, polls))
+
+    def set_prefill_rows(self, rows: int) -> None:
+        """Real rows a prefill chunk is filled up to past its `chunk` positions
+        (0: exactly `chunk` positions, whose rows then bound the workspace)."""
+        _check(lib().fmd_dec_set_prefill_rows(self.handle, rows))
 
     def op_layer_decode(self, caches: KvCache, layer: int, x_ptr: int, pad: Sequence[int],
                         batch: int) -> None:

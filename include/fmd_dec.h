@@ -86,6 +86,14 @@ void* fmd_dec_stream(const fmd_dec* dec);
  * 0 gives up at the first unmet poll (used by the tests of that path). */
 int fmd_dec_set_spin_limit(fmd_dec* dec, int polls);
 
+/* Real (non-pad) rows that a prefill chunk is filled up to: a chunk takes the
+ * caller's `chunk` positions, and more while they hold fewer than `rows` rows
+ * (default 12288).  0: exactly `chunk` positions, as the reference takes them
+ * (qwen3.rs:475-496), so that batch * chunk rows bound the prefill workspace
+ * (of the 0.6B shape, 12,288 rows take 0.6 GB).  Takes effect with the next
+ * prefill; workspace that earlier calls needed is kept. */
+int fmd_dec_set_prefill_rows(fmd_dec* dec, int rows);
+
 /* Loader::linear_with / fused_linear / get / build_tied_head
  * (linear.rs:166-265, qwen3.rs:355-372, 566-578).  `name` is the checkpoint
  * name (with or without "model.language_model."), e.g.
@@ -164,7 +172,7 @@ int fmd_dec_assemble(fmd_dec* dec, const uint32_t* ids, const int64_t* offsets, 
  * when embeds_on_device); pad[b] = left padding of row b.  Queries are taken
  * `chunk` positions at a time (the reference uses 256; pad rows are exactly
  * zero in the reference and are skipped), and more while those hold fewer than
- * 12,288 real rows.  Writes f32 logits (batch, vocab)
+ * 12,288 real rows (fmd_dec_set_prefill_rows).  Writes f32 logits (batch, vocab)
  * of each row's last position to `logits` (host) when non-NULL.  The cache
  * must be empty; its length becomes `total`. */
 int fmd_dec_prefill(fmd_dec* dec, fmd_kv* kv, const void* embeds, int embeds_on_device,

@@ -319,6 +319,30 @@ def test_prefill_chunks_by_rows(fmd, orc, prec, lens, chunk):
     assert np.array_equal(gpu.prefill(orc.to_storage(emb, OPREC[prec]), gkv, pad, chunk=chunk), got)
 
 
+def test_prefill_rows_bound_the_workspace(fmd):
+    """With set_prefill_rows(0) a caller's `chunk` bounds the prefill's device
+    memory again (8 x 64 rows against 8 x 1024 in one chunk: their workspaces are
+    a sixteenth apart, the fixed parts aside), and it can be set back."""
+    _announce("prefill rows and the workspace")
+    cfg = small_cfg(fmd, layers=1, vocab=256)
+    w = fmd.synthetic_weights(cfg, seed=44)
+    emb = torch.randn((8, 1024, 1024), generator=torch.Generator().manual_seed(45)).bfloat16().cuda()
+    used = {}
+    for rows in (0, None):
+        gpu = fmd.Qwen3(cfg, "bf16", max_len=1100).load(w)
+        kv = gpu.new_caches(8, 1040)
+        if rows is not None:
+            gpu.set_prefill_rows(rows)
+        torch.cuda.synchronize()
+        free = torch.cuda.mem_get_info()[0]
+        gpu.prefill_device(emb, kv, [0] * 8, 64)
+        used[rows] = free - torch.cuda.mem_get_info()[0]
+    print(f"[gap] workspace MiB {used[0] / 2**20:.0f} | {used[None] / 2**20:.0f}", flush=True)
+    assert used[0] * 2 < used[None]
+    with pytest.raises(fmd.FmdError, match="negative row count"):
+        gpu.set_prefill_rows(-1)
+
+
 # --------------------------------------------------------------------------
 # decode step over a synthetic padded context (configs 2 / 3 style)
 # --------------------------------------------------------------------------
