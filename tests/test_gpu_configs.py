@@ -106,6 +106,7 @@ def test_fp32_full_depth_prefill_and_greedy_vs_oracle(fmd, orc):
     gpu = fmd.Qwen3(cfg, "f32", max_len=T + budget + 8).load(w)
     ref = orc.OracleModel(cfg, OPREC["f32"], T + budget + 8).load(w)
     emb, pad = ref.padded_embeds(prompts)
+    gpu.set_prefill_rows(0)   # exactly 256 positions to a chunk
     gkv = gpu.new_caches(4, T + 4)
     got = gpu.prefill(emb, gkv, pad, chunk=256)
     del gkv

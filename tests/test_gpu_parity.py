@@ -556,6 +556,7 @@ def test_prefill_logits_and_cache(fmd, orc, prec, chunk):
     _announce(f"prefill {prec} chunk={chunk}")
     cfg = tiny_cfg(fmd)
     gpu, ref, w = build_pair(fmd, orc, cfg, prec, seed=61, max_len=2048)
+    gpu.set_prefill_rows(0)   # two chunks, and five
     rng = np.random.default_rng(62)
     prompts = [rng.integers(0, cfg.vocab_size, n).tolist() for n in (300, 41, 1, 257, 0, 128)]
     emb, pad = ref.padded_embeds(prompts)
@@ -585,19 +586,22 @@ def test_prefill_logits_and_cache(fmd, orc, prec, chunk):
 
 
 @pytest.mark.parametrize("heads,kv_heads", [(4, 4), (8, 2)])
-@pytest.mark.parametrize("chunk", [256, 64])
-def test_prefill_gqa_repeats(fmd, orc, heads, kv_heads, chunk):
-    """Prefill attention at GQA repeats 1 and 4 (the model runs at 2), bf16:
-    one-launch tiles (short key ranges) and split tiles (more than 256 keys)
-    against the oracle, logits and cache."""
-    _announce(f"prefill bf16 heads={heads} kv={kv_heads} chunk={chunk}")
+@pytest.mark.parametrize("prec,chunk", [("bf16", 256), ("bf16", 64), ("f16", 1024), ("f16", 256),
+                                        ("f16", 64), ("f32", 64)])
+def test_prefill_gqa_repeats(fmd, orc, heads, kv_heads, prec, chunk):
+    """Prefill attention at GQA repeats 1 and 4 (the model runs at 2): one-launch
+    tiles (short key ranges), split tiles (more than 256 keys; f16, which passes
+    over its keys once, more than 768) and their merge, and keys that an earlier
+    chunk cached, against the oracle, logits and cache."""
+    _announce(f"prefill {prec} heads={heads} kv={kv_heads} chunk={chunk}")
     cfg = fmd.TextConfig(vocab_size=1024, hidden_size=256, intermediate_size=512,
                          num_hidden_layers=2, num_attention_heads=heads,
                          num_key_value_heads=kv_heads, head_dim=128, rope_theta=1e6)
-    prec = "bf16"
     gpu, ref, w = build_pair(fmd, orc, cfg, prec, seed=67, max_len=2048)
+    gpu.set_prefill_rows(0)
     rng = np.random.default_rng(68)
-    prompts = [rng.integers(0, cfg.vocab_size, n).tolist() for n in (300, 41, 1, 257, 0, 128)]
+    longest = 900 if prec == "f16" else 300
+    prompts = [rng.integers(0, cfg.vocab_size, n).tolist() for n in (longest, 41, 1, 257, 0, 128)]
     emb, pad = ref.padded_embeds(prompts)
     B, T = len(prompts), emb.shape[1]
     gkv = gpu.new_caches(B, T + 8)
@@ -653,6 +657,7 @@ def test_kv_cache_indexing_bit_exact(fmd, orc, prec):
     _announce(f"kv indexing {prec}")
     cfg, w = _selection_model(fmd, seed=71)
     gpu, ref, _ = build_pair(fmd, orc, cfg, prec, weights=w, max_len=1024)
+    gpu.set_prefill_rows(0)   # three chunks
     rng = np.random.default_rng(72)
     prompts = [rng.integers(0, cfg.vocab_size, n).tolist() for n in (70, 3, 129, 1)]
     emb, pad = ref.padded_embeds(prompts)
@@ -685,11 +690,12 @@ def test_kv_cache_indexing_bit_exact(fmd, orc, prec):
 
 @pytest.mark.parametrize("prec", ["bf16", "f16"])
 @pytest.mark.parametrize("heads,kv_heads,lens,chunk", [
-    # 8 column groups of q|k|v: the 2460-row first chunk takes the 64-row
-    # direct-to-LDS tiles, the 940-row second chunk the register-staged ones
+    # 8 column groups of q|k|v: 64-row tiles for the 2460-row first chunk, 32-row
+    # ones for the 940-row second chunk
     (4, 2, (700, 690, 680, 670, 660), 512),
-    # 16 column groups: 128-row tiles at any row count
+    # 16 column groups: 32-row tiles, and at 3400 rows 128-row ones
     (8, 4, (300, 41, 129, 1), 256),
+    (8, 4, (700, 690, 680, 670, 660), 1024),
 ])
 def test_kv_cache_bit_exact_across_prefill_tiles(fmd, orc, prec, heads, kv_heads, lens, chunk):
     """The q|k|v projection's fused q/k norm + RoPE + cache-store epilogue in
@@ -701,6 +707,7 @@ def test_kv_cache_bit_exact_across_prefill_tiles(fmd, orc, prec, heads, kv_heads
     _announce(f"kv bit-exact {prec} heads={heads}/{kv_heads} lens={lens} chunk={chunk}")
     cfg, w = _selection_model(fmd, seed=73, heads=heads, kv_heads=kv_heads)
     gpu, ref, _ = build_pair(fmd, orc, cfg, prec, weights=w, max_len=1024)
+    gpu.set_prefill_rows(0)
     rng = np.random.default_rng(74)
     prompts = [rng.integers(0, cfg.vocab_size, n).tolist() for n in lens]
     emb, pad = ref.padded_embeds(prompts)
@@ -723,6 +730,7 @@ def test_kv_cache_bit_exact_across_prefill_tiles(fmd, orc, prec, heads, kv_heads
     cfg2 = tiny_cfg(fmd)
     cfg2.num_attention_heads, cfg2.num_key_value_heads = heads, kv_heads
     gpu, ref, w2 = build_pair(fmd, orc, cfg2, prec, seed=75, max_len=1024)
+    gpu.set_prefill_rows(0)
     emb, pad = ref.padded_embeds(prompts)
     g = gpu.prefill(orc.to_storage(emb, OPREC[prec]), gpu.new_caches(B, T + 2), pad, chunk=chunk)
     r = ref.prefill(ref.new_kv(B, T + 2), emb, pad)
