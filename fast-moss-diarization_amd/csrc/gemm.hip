@@ -357,6 +357,33 @@ __device__ __forceinline__ ResidRows<A, MI> load_resid(const GemmArgs& p, int m0
   return rr;
 }
 
+// EPI_RESID of the 64-row Q8_0 tiles and the 128-row dense ones: y = rd(resid +
+// rd(acc)), 2 bytes at a time, 16 lanes to 32 consecutive bytes of a row.  8-byte
+// pieces of the dense tiles' other layout, 16 rows to an instruction, are slower
+// (medians of five alternating runs, 2-byte | 8-byte, us, bf16): O at 12,288 rows
+// 66.7 | 68.9, 8000 42.0 | 43.2, 4800 33.0 | 35.3; down 87.3 | 90.7, 56.7 | 57.9,
+// 45.0 | 47.5; f16 at 6400 rows 36.6 | 39.1 and 52.0 | 54.4.
+template <int A, int BMT, int MI>
+__device__ __forceinline__ void resid_epilogue(const GemmArgs& p, const f32x4 (&acc)[MI][4], int m0,
+                                               const int (&tile)[4], const bool (&tv)[4],
+                                               const ResidRows<A, MI>& rr) {
+  typedef typename ActT<A>::T T;
+  const int lane = threadIdx.x & 63, wm = (threadIdx.x >> 6) >> 1;
+  const int row = lane & 15, kg = lane >> 4;
+#pragma unroll
+  for (int mi = 0; mi < MI; ++mi)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int gr = m0 + wm * (BMT / 2) + mi * 16 + 4 * kg + r;
+      if (gr >= p.M) continue;
+#pragma unroll
+      for (int ni = 0; ni < 4; ++ni)
+        if (tv[ni])
+          ((T*)p.y)[(size_t)gr * p.ldy + tile[ni] * 16 + row] =
+              st_act<A>(ld_act<A>(rr.v[mi][r][ni]) + rd<A>(acc[mi][ni][r]));
+    }
+}
+
 // EPI_SWIGLU epilogue (Mlp::forward's silu(gate) * up, qwen3.rs:288-291):
 // tiles 0, 1 of the wave hold gate columns, tiles 2, 3 the matching up
 // columns.  Each 16-row fragment's eight products are computed before any
@@ -539,7 +566,11 @@ gemm_q8_kernel(GemmArgs p) {
     swiglu_epilogue<A, BMT, MI>(p, acc, m0, tile, tv);
     return;
   }
-  // Epilogue.  Lane holds rows 4*kg + r of each 16-row fragment, column `row`.
+  if constexpr (EPI == EPI_RESID) {
+    resid_epilogue<A, BMT, MI>(p, acc, m0, tile, tv, rres);
+    return;
+  }
+  // EPI_STORE.  Lane holds rows 4*kg + r of each 16-row fragment, column `row`.
 #pragma unroll
   for (int mi = 0; mi < MI; ++mi) {
 #pragma unroll
@@ -547,14 +578,8 @@ gemm_q8_kernel(GemmArgs p) {
       const int gr = m0 + wm * (BMT / 2) + mi * 16 + 4 * kg + r;
       if (gr >= p.M) continue;
 #pragma unroll
-      for (int ni = 0; ni < 4; ++ni) {
-        if (!tv[ni]) continue;
-        const size_t o = (size_t)gr * p.ldy + tile[ni] * 16 + row;
-        if constexpr (EPI == EPI_RESID)
-          ((T*)p.y)[o] = st_act<A>(ld_act<A>(rres.v[mi][r][ni]) + rd<A>(acc[mi][ni][r]));
-        else
-          ((T*)p.y)[o] = st_act<A>(acc[mi][ni][r]);
-      }
+      for (int ni = 0; ni < 4; ++ni)
+        if (tv[ni]) ((T*)p.y)[(size_t)gr * p.ldy + tile[ni] * 16 + row] = st_act<A>(acc[mi][ni][r]);
     }
   }
 }
@@ -592,6 +617,11 @@ __device__ __forceinline__ uint32_t pack2_rounded(float lo, float hi) {
 // straight from the registers, and what is staged through LDS is written 8
 // bytes at a time.  Against 2-byte accesses in the other layout (the same
 // bits): encoder layer at 16 windows 936 -> 927 us, 5 x 1137 306.5 -> 304.4 us.
+// gate|up's stores from this layout, against 16-byte stores of products staged
+// through LDS (medians of five alternating runs, bf16): 12,288 rows 151.1 |
+// 148.2 us, 8000 100.3 | 99.9, 4800 64.2 | 65.8, 3200 50.2 | 50.1; f16 12,288
+// 155.6 | 154.5, 6400 95.4 | 96.2 -- within 2.5% either way, so not staged.
+// The 128-row residual tiles keep the other layout (resid_epilogue).
 
 // Four consecutive 16-bit values at q (VEC: 8-byte aligned).
 template <bool VEC>
@@ -818,6 +848,7 @@ gemm_dma_kernel(GemmArgs p) {
   typedef typename ActT<A>::T T;
   static_assert((BMT == 128 && NS == 4) || (BMT == 256 && NS == 3), "tile / ring");
   constexpr int MI = BMT / 32;           // 16-row fragments per wave
+  constexpr bool CROSS = EPI != EPI_RESID;   // the weights as the A operand
   constexpr int NX = BMT / 64;           // X copies per thread per stage
   constexpr int PER = NX + 2;            // copies per thread per stage
   constexpr int SA = BMT * BK2;          // X elements per stage
@@ -845,9 +876,9 @@ gemm_dma_kernel(GemmArgs p) {
     tv[ni] = (EPI == EPI_SWIGLU) ? (cg * 4 + wn * 2 + (ni & 1)) < ntiles / 2 : tile[ni] < ntiles;
   }
   const int mb = m0 + wm * (BMT / 2);
-  [[maybe_unused]] uint2 rres[MI][4];   // in flight behind the K loop
   static_assert(EPI != EPI_RESID || BMT <= 128, "residual prefetch: 128-row tiles");
-  if constexpr (EPI == EPI_RESID) cross_resid<true, MI, 4>(p, mb, tile, tv, rres);
+  [[maybe_unused]] ResidRows<A, EPI == EPI_RESID ? MI : 1> rres;   // in flight behind the K loop
+  if constexpr (EPI == EPI_RESID) rres = load_resid<A, BMT, MI>(p, m0, tile, tv);
   // This thread's copies per stage: X slots j * 64 + lane of instructions
   // j = NX w .. NX w + NX - 1 (rows 16 j + lane / 4; rows past M read row
   // M - 1), weight tiles t = 2w, 2w + 1 (past the end: the last tile).
@@ -911,7 +942,7 @@ gemm_dma_kernel(GemmArgs p) {
       const int r = wm * (BMT / 2) + mi * 16 + row;
       const u32x4 fa = *(const u32x4*)&a[(r * 4 + (kg ^ swz(r))) * 8];
 #pragma unroll
-      for (int ni = 0; ni < 4; ++ni) acc[mi][ni] = mfma16<A>(fb[ni], fa, acc[mi][ni]);
+      for (int ni = 0; ni < 4; ++ni) acc[mi][ni] = CROSS ? mfma16<A>(fb[ni], fa, acc[mi][ni]) : mfma16<A>(fa, fb[ni], acc[mi][ni]);
     }
   }
 
@@ -919,8 +950,11 @@ gemm_dma_kernel(GemmArgs p) {
     rope_epilogue<A, BMT, MI, true>(p, acc, smem, m0, cg, rrows);
   } else if constexpr (EPI == EPI_AFFINE) {
     staged_affine_epilogue<A, BMT, MI>(p, acc, m0, cg, smem);
+  } else if constexpr (EPI == EPI_RESID) {
+    resid_epilogue<A, BMT, MI>(p, acc, m0, tile, tv, rres);
   } else {
-    cross_epilogue<A, EPI, true, MI, 4>(p, acc, mb, tile, tv, rres);
+    const uint2 none[MI][4] = {};   // (read for a residual or a table only)
+    cross_epilogue<A, EPI, true, MI, 4>(p, acc, mb, tile, tv, none);
   }
 }
 
