@@ -642,7 +642,7 @@ int prefill_impl(fmd_dec* d, fmd_kv* kv, const void* emb_dev, const int32_t* pad
     // Items: split every tile's keys [pad_b, pos0 + n) into pieces of
     // `split` keys, with `split` chosen so the chunk's key blocks spread over
     // about kItemsPerHead items per KV head.  When every tile fits in one
-    // piece (short prompts), one launch runs both softmax passes.
+    // piece (short prompts), one launch does the whole attention.
     int nitems = 0;
     {
       long blocks = 0;

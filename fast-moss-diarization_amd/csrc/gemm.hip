@@ -745,13 +745,12 @@ __device__ __forceinline__ void cross_epilogue(const GemmArgs& p, const f32x4 (&
 
 // EPI_AFFINE on the direct-to-LDS BMT x 128 tiles, through LDS: the
 // accumulators, rounded to the activation dtype (the first affine step), are
-// staged row-major in the freed ring -- the 16-byte chunk c of tile row R at
-// chunk position c ^ rope_sw(R), so the 2-byte writes of a wave's four
-// 16-lane groups (rows 4 apart) fall in distinct banks and a row's 16 chunk
-// reads cover all of them -- then 16 lanes per row finish 8 columns each,
-// two rows per pass (16 independent chains through affine_block), with
-// 16-byte residual and table loads and 16-byte stores instead of 2-byte
-// accesses in the accumulators' layout.
+// staged row-major in the freed ring, 8 bytes (four columns) at a time -- the
+// 16-byte chunk c of tile row R at chunk position c ^ (R & 15) -- then 16 lanes
+// per row finish 8 columns each, two rows per pass (16 independent chains through
+// affine_block), with 16-byte residual and table loads and 16-byte stores: 8-byte
+// stores straight from the accumulators cost the 128- and 256-row tiles 17-20%
+// (fc1 at 16 windows 243 -> 283 us, q|k|v 167 -> 200).
 template <int A, int BMT, int MI>
 __device__ __forceinline__ void staged_affine_epilogue(const GemmArgs& p, const f32x4 (&acc)[MI][4], int m0,
                                                        int cg, uint16_t* stg) {
@@ -959,21 +958,21 @@ gemm_dma_kernel(GemmArgs p) {
 }
 
 // ---------------------------------------------------------------------------
-// Small grids: BM x BN tiles (32 or 64 rows x 32, 64 or 128 columns), four
+// Small grids: BM x BN tiles (32, 64 or 128 rows x 32, 64 or 128 columns), four
 // waves in 2 x 2 (BM/2 x BN/2 each), for products whose 64 x 128 tiles would
 // leave most CUs without a work-group.
 //
-// What bounds them is the serial K loop of one work-group, not bytes: the
-// 64 x 128 register-staged tiles took 23 us for K = 3072 at any M up to 2048
-// (32 work-groups on 256 CUs at M = 256), the 33 us of Q8_0 likewise.  A
+// What bounds them is the serial K loop of one work-group, not bytes: 64 x 128
+// register-staged tiles, which ran them before, took 23 us for K = 3072 at any M
+// up to 2048 (32 work-groups on 256 CUs at M = 256), Q8_0 ones 33 us.  A
 // smaller tile has less to copy, read and multiply per k and the ring keeps
 // 30-70 KB of it in flight per work-group: 7.6 us (dense, 32 x 32) and 11.8 us
 // (Q8_0) at M = 256, N = 1024, K = 3072 (try_small has the rule and figures).
 //
 // Both operands (for Q8_0 the quants and the scales too) go global -> LDS by
 // direct-to-LDS loads through a ring of NS stages of KS k, NS - 1 in flight,
-// one barrier per stage.  KS is 64 for dense weights and 128 for Q8_0 (a
-// stage is then a whole number of copies per wave).  X stage: row r is KS / 8
+// one barrier per stage.  KS is 64 or 128 for dense weights and 128 or 256 for
+// Q8_0 (a stage is then a whole number of copies per wave).  X stage: row r is KS / 8
 // chunks of 16 bytes, chunk c at position c ^ swx(r), so that the fragment
 // reads (16 rows, one chunk) fall in distinct banks.  Weight stage: the tiles'
 // fragments as stored; Q8_0 scales: 16 x 2 u32 per tile.  Each output is
@@ -1281,15 +1280,20 @@ __global__ void __launch_bounds__(256) gemm32_kernel(GemmArgs p) {
 }
 
 // Rows of the 16-bit dense tiles past the small grids (512 work-groups = two
-// per CU), chosen from bf16 sweeps over the prefill shapes and row counts: 256
-// where those tiles fill about 4/5 of the slots and do not end in a last round
-// of fewer than 128 work-groups (qkv M = 3584 36.5 against 38.9 us, M = 4096
-// 39.2 against 42.4; down M = 13509, 424 tiles, 95.5 against 108.6, but M =
-// 12008, 376 tiles, 90.2 against 86.1; gate|up M = 2560 38.0 against 41.4, but
-// M = 3072, 576 tiles, 56.2 against 51.9), else 128 (64-row tiles, which
-// narrow outputs took up to 512 tiles of 128 rows, were slower past the small
-// grids: O M = 4503 33.8 against 31.3 us, M = 7505 44.8 against 37.0; down
-// 47.7 against 43.3 and 66.2 against 53.3).
+// per CU): 256 where those tiles fill about 4/5 of the slots and do not end in a
+// last round of fewer than 128 work-groups, else 128.  It decides for gate|up,
+// the encoder's products and plain stores; q|k|v with its RoPE epilogue and the
+// residual products of the decoder take 128 rows wherever it says 256 (dispatch).
+// us, 256 | 128 rows, bf16, by tiles of 256 rows:
+//   gate|up at 2240 rows (432 tiles) 36.4 | 37.4, 2560 (480) 36.6 | 40.0, but
+//   3072 (576) 52.5 | 48.9; 4096 (768) 56.3 | 59.5, 12,288 (2304) 158.1 | 178.3;
+//   the encoder's fc1 at 3300 (416) 43.7 | 44.9, 4500 (576) 64.0 | 60.9, 12,000
+//   (1504) 128.9 | 147.4; its q|k|v at 3300 (312) 37.6 | 35.2, 4500 (432) 39.8 |
+//   41.9, 24,000 (2256) 165.6 | 198.0; its fc2 at 12,000 (376) 119.5 | 118.3,
+//   14,000 (440) 125.5 | 141.2, 18,000 (568) 187.5 | 176.7.
+// (64-row tiles were slower than 128-row ones past the small grids: O at 4503
+// rows 33.8 against 31.3, 7505 44.8 against 37.0; down 47.7 against 43.3 and 66.2
+// against 53.3.)
 int gemm_tile_rows(int M, int col_groups) {
   const int tiles256 = (M + 255) / 256 * col_groups;
   return tiles256 >= 400 && (tiles256 % 512 == 0 || tiles256 % 512 >= 128) ? 256 : 128;
@@ -1335,7 +1339,7 @@ hipError_t launch_q8(int epi, dim3 grid, const GemmArgs& a, hipStream_t s) {
 // XCD rows a (1, 2, 4 or 8; the XCD grid is a x 8/a) for an M x N x K
 // product: the X bytes are fetched 8/a times and the weight bytes a times;
 // the column groups must split evenly over 8/a.
-int xcd_rows(const GemmArgs& p, int cols, int bm) {
+int xcd_rows(const GemmArgs& p, int cols) {
   const double xb = (double)p.M * p.W.in * 2;
   const double wb = (double)p.W.out * p.W.in * (p.W.kind == WK_Q8 ? 34.0 / 32 : 2.0);
   int best = 1;
@@ -1345,7 +1349,6 @@ int xcd_rows(const GemmArgs& p, int cols, int bm) {
     const double c = (8 / a) * xb + a * wb;
     if (c < cost) cost = c, best = a;
   }
-  (void)bm;
   return best;
 }
 
@@ -1355,7 +1358,7 @@ hipError_t launch_small(int epi, const GemmArgs& a, hipStream_t s) {
   const int cw = epi == EPI_SWIGLU ? BN / 32 : BN / 16;
   const int cols = ((epi == EPI_SWIGLU ? ntiles / 2 : ntiles) + cw - 1) / cw;
   GemmArgs g = a;
-  g.map = xcd_rows(a, cols, BM);
+  g.map = xcd_rows(a, cols);
   const int mtiles = (a.M + BM - 1) / BM, Ma = (mtiles + g.map - 1) / g.map;
   const dim3 grid(8 * Ma * (cols / (8 / g.map)));
 #define SMALL(E) hipLaunchKernelGGL((gemm_small_kernel<A, WK, E, BM, BN, KS, NS, VEC>), grid, dim3(256), 0, s, g)
@@ -1453,7 +1456,7 @@ hipError_t dispatch(int epi, const GemmArgs& a, hipStream_t s) {
     // not fit its registers: 128-row tiles instead
     if ((epi == EPI_ROPE || epi == EPI_RESID) && bm == 256) bm = 128;
     GemmArgs g = a;
-    g.map = xcd_rows(a, cols, bm);
+    g.map = xcd_rows(a, cols);
     const int mtiles = (a.M + bm - 1) / bm, Ma = (mtiles + g.map - 1) / g.map;
     const dim3 grid(8 * Ma * (cols / (8 / g.map)));
     if constexpr (WK == WK_Q8) return launch_q8(epi, grid, g, s);

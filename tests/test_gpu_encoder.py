@@ -284,9 +284,10 @@ def test_encoder_argument_errors(fmd):
 
 
 def test_windows_are_independent_of_the_batch(fmd, orc):
-    """Twelve windows at Whisper-medium width in one pass (18,012 rows, all
-    in 256-row tiles) against each window alone (1,501 rows: 128- and 64-row
-    tiles): the same bits, since every tile kind sums each output over k in
+    """Twelve windows at Whisper-medium width in one pass (18,012 rows: 256-row
+    tiles for q|k|v and fc1, 128-row ones for out and fc2) against each window
+    alone (1,501 rows: 128-row tiles, and 64 x 64 small-grid ones for out and
+    fc2): the same bits, since every tile kind sums each output over k in
     the same order, applies the same epilogue steps (the residual ones
     included), and nothing crosses a window."""
     print("[gpu] encoder batch independence (tile kinds)", flush=True)
