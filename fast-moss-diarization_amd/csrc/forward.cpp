@@ -517,7 +517,8 @@ namespace {
 // from the reference's rounding, bar 0.02: 2048 .0215, 4096 .0176, 8192 .0234,
 // 12288 .0195, 16384 .0215; rms .0049 at each).
 // Which rows share a chunk changes no row's products, and its attention only in
-// where the keys are cut into items.
+// where the keys are cut into items (bf16: the order of f32 sums; f16: also the
+// reference that each item's probabilities are rounded against).
 int chunk_positions(const int32_t* pad, int B, int start, int total, int chunk, int fill) {
   int end = start + std::min(chunk, total - start);
   int64_t rows = 0;
@@ -949,9 +950,12 @@ extern "C" int fmd_dec_generate(fmd_dec* d, const void* embeds, int on_dev, cons
   if (chunk <= 0) chunk = 256;
   // new_caches(batch, max_prompt + budget) (engine.rs:470, 493).  A batch of
   // more than kMaxDecodeRows rows runs as groups of at most that many rows
-  // over the same padded length: each row's tokens depend only on its own
-  // padded prompt (the kernels' per-row reductions do not depend on the
-  // batch), so they are the tokens of the whole batch run at once.
+  // over the same padded length.  A row's tokens depend on its own padded prompt
+  // alone up to rounding: products and norms give a row the same bits in any
+  // batch, but attention sums a row's keys in pieces whose length comes from the
+  // whole batch (decode: its rows and the cache's capacity; 16-bit prefill over
+  // more than 256 keys, f16 768: the rows of the chunk), which can move a logit by
+  // an ulp or two of the activation dtype.
   const size_t row_bytes = (size_t)total * d->H * d->esz;
   for (int g0 = 0; g0 < B; g0 += kMaxDecodeRows) {
     const int n = std::min(kMaxDecodeRows, B - g0);

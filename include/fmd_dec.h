@@ -190,8 +190,11 @@ int fmd_dec_decode_step(fmd_dec* dec, fmd_kv* kv, const uint32_t* ids, const int
  * ntok[b] tokens kept per row; finish[b]: 0 = Length, 1 = Stop.
  * force_eot_step (may be NULL): row b's argmax is replaced by eos at greedy
  * step force_eot_step[b] (synthetic end-of-turn).  Any batch size: above 16
- * rows, groups of 16 rows run one after another over the same padded length,
- * which gives each row the tokens of one batched run.  Decode positions come
+ * rows, groups of 16 rows run one after another over the same padded length.
+ * A row's logits do not depend on its batch-mates but for rounding: attention
+ * sums a row's keys in pieces cut for the whole batch, which can move a logit by
+ * an ulp or two of the activation dtype, and with it a token whose two best
+ * logits are that close.  Decode positions come
  * from the RoPE table (max_len of fmd_dec_create): if rows are still
  * generating when position max_len would be written, the call fails, as the
  * reference's decode_step does at Rope::apply (qwen3.rs:139-144). */

@@ -797,7 +797,8 @@ def test_host_loop_with_device_greedy_matches_device_loop(fmd, orc):
 
 def test_batched_equals_solo(fmd, orc):
     """python/tests/test_engine.py:148-173 made exact: a row's greedy tokens
-    do not depend on its batch-mates (same left padding)."""
+    do not depend on its batch-mates (same left padding; prompts of one
+    attention item)."""
     _announce("batched vs solo")
     cfg = tiny_cfg(fmd)
     gpu, _, _ = build_pair(fmd, orc, cfg, "int8", seed=91, max_len=1024)
@@ -807,6 +808,39 @@ def test_batched_equals_solo(fmd, orc):
     for i, p in enumerate(prompts):
         solo = gpu.generate_batch([p], 16, eos=5)[0]
         assert solo.tokens == batched[i].tokens
+
+
+@pytest.mark.parametrize("prec", PRECS)
+def test_long_prompts_batched_against_solo(fmd, prec):
+    """Prompts long enough for split attention tiles, each alone and in a batch
+    of eight (other cut points of its keys): f32 logits and every precision's
+    layer-0 cache are the same bits; 16-bit logits within two ulps of the
+    activation dtype at the row's largest one -- each logit's own rounding, of a
+    value that moved less than half an ulp, can turn one; the layers' flipped
+    roundings that reach it are allowed another."""
+    _announce(f"long prompts batched vs solo {prec}")
+    cfg = tiny_cfg(fmd)
+    gpu = fmd.Qwen3(cfg, prec, max_len=3100).load(fmd.synthetic_weights(cfg, seed=91))
+    dt = {"f32": torch.float32, "bf16": torch.bfloat16}.get(prec, torch.float16)
+    T, pad = 3000, [0, 1500, 100, 700, 2999, 2000, 10, 2300]
+    emb = torch.randn((8, T, cfg.hidden_size), generator=torch.Generator().manual_seed(1)).to(dt).cuda()
+    for b, p in enumerate(pad):
+        emb[b, :p] = 0
+    torch.cuda.synchronize()
+    kv = gpu.new_caches(8, T)
+    batched = gpu.prefill_device(emb, kv, pad, 512)
+    caches = [kv.read(0, which) for which in (0, 1)]
+    for b, p in enumerate(pad):
+        one, kv1 = emb[b:b + 1].contiguous(), gpu.new_caches(1, T)
+        torch.cuda.synchronize()
+        solo = gpu.prefill_device(one, kv1, [p], 512)[0]
+        for which in (0, 1):
+            assert np.array_equal(kv1.read(0, which)[0], caches[which][b]), (b, which)
+        top = float(np.abs(solo).max())
+        bar = 0.0 if prec == "f32" else 2.0 * 2.0 ** (np.floor(np.log2(top)) - (7 if prec == "bf16" else 10))
+        d = float(np.abs(solo - batched[b]).max())
+        print(f"[gap] solo {prec} row {b}: {d:.3g} of {bar:.3g}", flush=True)
+        assert d <= bar, (b, d, bar)
 
 
 def test_engine_sorts_and_chunks(fmd, orc):
