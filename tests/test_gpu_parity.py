@@ -290,6 +290,7 @@ def test_layer_decode_on_unaligned_rows_and_moved_lengths(fmd, prec, B):
 @pytest.mark.parametrize("prec,lens,chunk", [
     ("f16", (3000, 1, 1100, 2500) + (900,) * 8, 64),     # 13,801 rows: two chunks
     ("int8", (2049,) * 6, 256),                          # one chunk of 12,288 rows and one of 6
+    ("f32", (1700, 3) + (1601,) * 7, 256),               # 12,910 rows: two chunks
     ("bf16", (3300, 1000, 3300, 200, 3299, 3300), 2000), # `chunk` positions hold more at the end
 ])
 def test_prefill_chunks_by_rows(fmd, orc, prec, lens, chunk):
