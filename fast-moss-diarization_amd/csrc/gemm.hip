@@ -384,6 +384,29 @@ __device__ __forceinline__ void resid_epilogue(const GemmArgs& p, const f32x4 (&
     }
 }
 
+// EPI_STORE of the 64-row Q8_0 tiles and the 128- and 256-row dense ones, in the
+// same layout, to any alignment.  Against 8-byte pieces of the other layout (us,
+// medians of four alternating runs, bf16): K = 1024, N = 6144 at 3200 rows 51.5 |
+// 54.8, 6000 90.8 | 96.5, 12,288 174.3 | 185.8, 24,016 331.9 | 351.7; N = 4096
+// 36.8 | 38.2, 58.8 | 60.5, 115.0 | 122.0, 257.4 | 262.1.
+template <int A, int BMT, int MI>
+__device__ __forceinline__ void store_epilogue(const GemmArgs& p, const f32x4 (&acc)[MI][4], int m0,
+                                               const int (&tile)[4], const bool (&tv)[4]) {
+  typedef typename ActT<A>::T T;
+  const int lane = threadIdx.x & 63, wm = (threadIdx.x >> 6) >> 1;
+  const int row = lane & 15, kg = lane >> 4;
+#pragma unroll
+  for (int mi = 0; mi < MI; ++mi)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int gr = m0 + wm * (BMT / 2) + mi * 16 + 4 * kg + r;
+      if (gr >= p.M) continue;
+#pragma unroll
+      for (int ni = 0; ni < 4; ++ni)
+        if (tv[ni]) ((T*)p.y)[(size_t)gr * p.ldy + tile[ni] * 16 + row] = st_act<A>(acc[mi][ni][r]);
+    }
+}
+
 // EPI_SWIGLU epilogue (Mlp::forward's silu(gate) * up, qwen3.rs:288-291):
 // tiles 0, 1 of the wave hold gate columns, tiles 2, 3 the matching up
 // columns.  Each 16-row fragment's eight products are computed before any
@@ -570,18 +593,7 @@ gemm_q8_kernel(GemmArgs p) {
     resid_epilogue<A, BMT, MI>(p, acc, m0, tile, tv, rres);
     return;
   }
-  // EPI_STORE.  Lane holds rows 4*kg + r of each 16-row fragment, column `row`.
-#pragma unroll
-  for (int mi = 0; mi < MI; ++mi) {
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int gr = m0 + wm * (BMT / 2) + mi * 16 + 4 * kg + r;
-      if (gr >= p.M) continue;
-#pragma unroll
-      for (int ni = 0; ni < 4; ++ni)
-        if (tv[ni]) ((T*)p.y)[(size_t)gr * p.ldy + tile[ni] * 16 + row] = st_act<A>(acc[mi][ni][r]);
-    }
-  }
+  store_epilogue<A, BMT, MI>(p, acc, m0, tile, tv);
 }
 
 // 16-bit activations with dense 16-bit weights, both operands copied global
@@ -621,7 +633,8 @@ __device__ __forceinline__ uint32_t pack2_rounded(float lo, float hi) {
 // through LDS (medians of five alternating runs, bf16): 12,288 rows 151.1 |
 // 148.2 us, 8000 100.3 | 99.9, 4800 64.2 | 65.8, 3200 50.2 | 50.1; f16 12,288
 // 155.6 | 154.5, 6400 95.4 | 96.2 -- within 2.5% either way, so not staged.
-// The 128-row residual tiles keep the other layout (resid_epilogue).
+// Residuals and plain stores of the 128- and 256-row tiles keep the other layout
+// (resid_epilogue, store_epilogue).
 
 // Four consecutive 16-bit values at q (VEC: 8-byte aligned).
 template <bool VEC>
@@ -847,7 +860,7 @@ gemm_dma_kernel(GemmArgs p) {
   typedef typename ActT<A>::T T;
   static_assert((BMT == 128 && NS == 4) || (BMT == 256 && NS == 3), "tile / ring");
   constexpr int MI = BMT / 32;           // 16-row fragments per wave
-  constexpr bool CROSS = EPI != EPI_RESID;   // the weights as the A operand
+  constexpr bool CROSS = EPI != EPI_RESID && EPI != EPI_STORE;   // weights as the A operand
   constexpr int NX = BMT / 64;           // X copies per thread per stage
   constexpr int PER = NX + 2;            // copies per thread per stage
   constexpr int SA = BMT * BK2;          // X elements per stage
@@ -941,7 +954,8 @@ gemm_dma_kernel(GemmArgs p) {
       const int r = wm * (BMT / 2) + mi * 16 + row;
       const u32x4 fa = *(const u32x4*)&a[(r * 4 + (kg ^ swz(r))) * 8];
 #pragma unroll
-      for (int ni = 0; ni < 4; ++ni) acc[mi][ni] = CROSS ? mfma16<A>(fb[ni], fa, acc[mi][ni]) : mfma16<A>(fa, fb[ni], acc[mi][ni]);
+      for (int ni = 0; ni < 4; ++ni)
+        acc[mi][ni] = CROSS ? mfma16<A>(fb[ni], fa, acc[mi][ni]) : mfma16<A>(fa, fb[ni], acc[mi][ni]);
     }
   }
 
@@ -951,7 +965,9 @@ gemm_dma_kernel(GemmArgs p) {
     staged_affine_epilogue<A, BMT, MI>(p, acc, m0, cg, smem);
   } else if constexpr (EPI == EPI_RESID) {
     resid_epilogue<A, BMT, MI>(p, acc, m0, tile, tv, rres);
-  } else {
+  } else if constexpr (EPI == EPI_STORE) {
+    store_epilogue<A, BMT, MI>(p, acc, m0, tile, tv);
+  } else {   // EPI_SWIGLU
     const uint2 none[MI][4] = {};   // (read for a residual or a table only)
     cross_epilogue<A, EPI, true, MI, 4>(p, acc, mb, tile, tv, none);
   }
@@ -1416,9 +1432,12 @@ bool try_small(int epi, const GemmArgs& a, hipStream_t s, hipError_t* e) {
     else return false;
   } else {
     // a caller's unaligned output (EPI_STORE only: every other product works on
-    // the library's buffers) is stored element by element, by one tile kind
-    if (epi == EPI_STORE && !vec_ok(a)) *e = launch_small<A, WK, 128, 64, 64, 3, false>(epi, a, s);
-    else if (epi != EPI_ROPE && !vec_ok(a)) *e = hipErrorInvalidValue;
+    // the library's buffers) is stored element by element, by one kind of small
+    // tile, and past it by the larger tiles, which always store so
+    if (epi == EPI_STORE && !vec_ok(a)) {
+      if (!fits(128, 64, 64, 512)) return false;
+      *e = launch_small<A, WK, 128, 64, 64, 3, false>(epi, a, s);
+    } else if (epi != EPI_ROPE && !vec_ok(a)) *e = hipErrorInvalidValue;
     else if (n32 && fits(32, 32, 128, 256)) *e = launch_small<A, WK, 32, 32, 128, 4>(epi, a, s);
     else if (n64 && fits(32, 64, 128, 256)) *e = launch_small<A, WK, 32, 64, 128, 3>(epi, a, s);
     else if (n64 && fits(64, 64, 128, 256)) *e = launch_small<A, WK, 64, 64, 128, 3>(epi, a, s);
